@@ -575,9 +575,7 @@ __global__ void zero_counters_kernel(unsigned long long *c) {
 
 static size_t stack_bytes(int block) { return size_t(kLdsWordsPerThread) * block * sizeof(int); }
 
-// Blocks of `kern` the current device holds at once (compute units x
-// resident blocks per unit), cached per (device, kernel, block size).
-static unsigned resident_grid(const void *kern, int block) {
+unsigned resident_grid(const void *kern, int block, size_t lds) {
   static std::mutex mu;
   static std::map<std::tuple<int, const void *, int>, unsigned> cache;
   int dev = 0;
@@ -588,7 +586,7 @@ static unsigned resident_grid(const void *kern, int block) {
   if (it != cache.end()) return it->second;
   int cus = 0, per_cu = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, stack_bytes(block));
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, lds);
   const unsigned g = unsigned(std::max(1, per_cu) * std::max(1, cus));
   cache[key] = g;
   return g;
@@ -676,6 +674,23 @@ static int log_tile() {
   return tile;
 }
 
+// Whether the one-box volume tracker takes a launch of integrator d on scene
+// s (an explicit samples_per_thread asks for the static launch).
+static bool takes_box(const Scene *s, const rcv_integrator_desc *d) {
+  return d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && d->max_depth != 0 && s->box_path();
+}
+
+// Work-unit split of the one-box renders: up to 64 units per pixel of at
+// least kVolUnitSamples samples, within the unit-sum buffer (floats per
+// unit: `words`).
+static int box_chunk_log2(const Scene *s, int64_t n_pix, int spp, int static_cl2, int words) {
+  int cl2 = 0;
+  while (cl2 < 6 && ((n_pix << (cl2 + 1)) * words) <= s->partial_cap &&
+         ((spp >> (cl2 + 1)) >= kVolUnitSamples || (cl2 < static_cl2 && (2 << cl2) <= spp)))
+    ++cl2;
+  return cl2;
+}
+
 // Work-unit split of a persistent volume launch: the chunk count of the
 // static launch (enough units to fill the device), raised while a unit keeps
 // at least min_samples samples.
@@ -725,6 +740,12 @@ static int check_states(const Scene *s, int ns, const char *fn) {
     if (int rc = need(m.albedo_param, "albedo")) return rc;
   }
   return RCV_OK;
+}
+
+static GradTargets no_targets() {
+  GradTargets g;
+  g.clear();
+  return g;
 }
 
 struct RenderLaunch {
@@ -801,7 +822,20 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
   const unsigned grid = ceil_div(threads, block);
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
   const RenderLaunch L{dim3(grid), block, stream, &s->view, I, sensor, seed, spp, spt, cl2, img_old, img_new};
-  if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE) {
+  if (takes_box(s, d)) {
+    const int ucl2 = box_chunk_log2(s, n_pix, spp, cl2, 3 * ns);
+    const GradTargets none = no_targets();
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    launch_box(s, ns, kBoxRender,
+               BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), nullptr, &none,
+                         s->partial, s->work_queue});
+    if (ns == 2)
+      hipLaunchKernelGGL(reduce_units_kernel<2>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+                         ucl2, spp, img_old, img_new);
+    else
+      hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+                         ucl2, spp, img_old, img_new);
+  } else if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE) {
     with_volume_features(s->features(), [&](auto f) {
       launch_render_kernel<1, RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>(L);
     });
@@ -815,7 +849,7 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
     RCV_REQUIRE(int64_t(units) * 3 * ns <= s->partial_cap, "%s: unit buffer too small", fn);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
     auto go = [&](auto kern) {
-      const unsigned pgrid = std::min(resident_grid(reinterpret_cast<const void *>(kern), block), grid);
+      const unsigned pgrid = std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)), grid);
       hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
                          ucl2, s->partial, s->work_queue, units);
     };
@@ -840,6 +874,57 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
       launch_render_kernel<1, RCV_INTEGRATOR_PATH, 0>(L);
   }
   return check_launch(fn);
+}
+
+// The scatter log of a persistent volume adjoint (buf, for the gradient of
+// `param`; -1: none, the scatter-adds stay atomics).
+struct LogLaunch {
+  LogBuf buf;
+  int param = -1;
+  int tile = 0;
+  int64_t nvox = 0;
+};
+
+// The density gradient of the first heterogeneous medium that has one goes
+// through the scatter log when its grid fits the reduction tiles and a
+// footprint (up to nx ny + nx + 1 voxels past its base) spans at most two
+// of them. Without memory for the log the scatter-adds stay atomics.
+static void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL) {
+  log.tile = log_tile();
+  for (const MediumInfo &M : s->media) {
+    if (M.homogeneous || M.sigma_param < 0 || !G.g[M.sigma_param]) continue;
+    const Param &P = s->params[M.sigma_param];
+    const int64_t n = int64_t(P.nx) * P.ny * P.nz;
+    if (n <= int64_t(log.tile) * kLogMaxTiles && n < (int64_t(1) << kRecBaseBits) &&
+        int64_t(P.nx) * P.ny + P.nx + 1 <= log.tile) {
+      log.param = M.sigma_param;
+      log.nvox = n;
+    }
+    break;
+  }
+  if (log.param >= 0 && log_buffer(stream, log.buf) != RCV_OK) {
+    (void)hipGetLastError();
+    log.param = -1;
+  }
+  if (log.param < 0) return;
+  GL.log_rec = log.buf.rec;
+  GL.log_ctl = log.buf.ctl;
+  GL.log_list = log.buf.list;
+  GL.log_fill = log.buf.fill;
+  GL.log_chunks = log_pool_chunks();
+  GL.log_shift = __builtin_ctz(unsigned(log.tile));
+  GL.log_param = log.param;
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1 + kLogBins), 0, stream, log.buf.ctl);
+}
+
+static void reduce_log(const Scene *s, const GradTargets &GL, hipStream_t stream, const LogLaunch &log) {
+  if (log.param < 0) return;
+  const Param &P = s->params[log.param];
+  const int tiles = int((log.nvox + log.tile - 1) / log.tile);
+  hipLaunchKernelGGL(log_reduce_kernel, dim3(kLogSplits, tiles), dim3(kReduceBlock),
+                     size_t(log.tile) * sizeof(long long), stream, log.buf.rec, log.buf.ctl, log.buf.list,
+                     log.buf.fill, GL.log_chunks, int(P.nx), int(P.nx) * int(P.ny), log.nvox, log.tile,
+                     GL.g[log.param]);
 }
 
 int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uint32_t seed, int spp,
@@ -879,7 +964,7 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     const int ucl2 = unit_chunk_log2(spp, cl2, kAdjUnitSamples);
     const unsigned units = unsigned(n_pix << ucl2);
     const unsigned pgrid =
-        std::min(resident_grid(reinterpret_cast<const void *>(kern), block), ceil_div(int64_t(units), block));
+        std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)), ceil_div(int64_t(units), block));
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
     hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp, ucl2,
                        grad_img, G, s->work_queue, units);
@@ -894,75 +979,42 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
                          dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp, spt, cl2, grad_img,
                          G);
     });
-  else if (d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread)
-    with_render_features(s->features(), [&](auto f) {
-      // the waves that fit, pulling units of >= kVolUnitSamples samples
-      // (fewer where the image is too small to fill the device otherwise)
-      constexpr int F = decltype(f)::value;
-      // (taped kernels keep kAdjUnitSamples: their per-lane tape in scratch
-      // gains nothing from coherence; the 64^3 k = 8 adjoint took 59.4 ms
-      // with 2-sample units against 51.2 ms)
-      const int ucl2 = unit_chunk_log2(spp, cl2, kTapeAdjoint<F> ? kAdjUnitSamples : kVolUnitSamples);
-      const unsigned units = unsigned(n_pix << ucl2);
-      // the density gradient of the first heterogeneous medium that has one
-      // goes through the scatter log when its grid fits the reduction tiles
-      // and a footprint (up to nx ny + nx + 1 voxels past its base) spans
-      // at most two of them
-      GradTargets GL = G;
-      int lp = -1;
-      int64_t nvox = 0;
-      const int tile = log_tile();
-      if constexpr (!kTapeAdjoint<F>) {
-        for (const MediumInfo &M : s->media) {
-          if (M.homogeneous || M.sigma_param < 0 || !G.g[M.sigma_param]) continue;
-          const Param &P = s->params[M.sigma_param];
-          const int64_t n = int64_t(P.nx) * P.ny * P.nz;
-          if (n <= int64_t(tile) * kLogMaxTiles && n < (int64_t(1) << kRecBaseBits) &&
-              int64_t(P.nx) * P.ny + P.nx + 1 <= tile) {
-            lp = M.sigma_param;
-            nvox = n;
-          }
-          break;
-        }
-      }
-      LogBuf lb;
-      // without memory for the log the scatter-adds stay atomics
-      if (lp >= 0 && log_buffer(stream, lb) != RCV_OK) {
-        (void)hipGetLastError();
-        lp = -1;
-      }
-      if (lp >= 0) {
-        GL.log_rec = lb.rec;
-        GL.log_ctl = lb.ctl;
-        GL.log_list = lb.list;
-        GL.log_fill = lb.fill;
-        GL.log_chunks = log_pool_chunks();
-        GL.log_shift = __builtin_ctz(unsigned(tile));
-        GL.log_param = lp;
-        hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1 + kLogBins), 0, stream, lb.ctl);
-      }
-      // three waves per SIMD with the log, four with atomics (kWavesPerEuLoggedAdjoint)
-      auto go = [&](auto kern) {
-        const unsigned pgrid =
-            std::min(resident_grid(reinterpret_cast<const void *>(kern), block), ceil_div(int64_t(units), block));
-        hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
-        hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
-                           ucl2, grad_img, GL, s->work_queue, units);
-      };
-      if constexpr (kTapeAdjoint<F>)
-        go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
-      else if (lp >= 0)
-        go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint>);
-      else
-        go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
-      if (lp >= 0) {
-        const Param &P = s->params[lp];
-        const int tiles = int((nvox + tile - 1) / tile);
-        hipLaunchKernelGGL(log_reduce_kernel, dim3(kLogSplits, tiles), dim3(kReduceBlock), size_t(tile) * sizeof(long long),
-                           stream, lb.rec, lb.ctl, lb.list, lb.fill, GL.log_chunks, int(P.nx),
-                           int(P.nx) * int(P.ny), nvox, tile, G.g[lp]);
-      }
-    });
+  else if (d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread) {
+    const bool box = takes_box(s, d);
+    const bool taped = !box && (s->features() & kFeatSupergrid) && !(s->features() & kFeatAlbedoGrid);
+    // (taped kernels keep kAdjUnitSamples: their per-lane tape in scratch
+    // gains nothing from coherence; the 64^3 k = 8 adjoint took 59.4 ms
+    // with 2-sample units against 51.2 ms)
+    const int ucl2 = unit_chunk_log2(spp, cl2, taped ? kAdjUnitSamples : kVolUnitSamples);
+    const unsigned units = unsigned(n_pix << ucl2);
+    GradTargets GL = G;
+    LogLaunch log;
+    if (!taped) open_log(s, G, stream, log, GL);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    if (box)
+      launch_box(s, 1, kBoxAdjoint,
+                 BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, units, grad_img, &GL, nullptr, s->work_queue});
+    else
+      with_render_features(s->features(), [&](auto f) {
+        // the waves that fit, pulling units of >= kVolUnitSamples samples
+        // (fewer where the image is too small to fill the device otherwise)
+        constexpr int F = decltype(f)::value;
+        auto go = [&](auto kern) {
+          const unsigned pgrid = std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)),
+                                          ceil_div(int64_t(units), block));
+          hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
+                             ucl2, grad_img, GL, s->work_queue, units);
+        };
+        // three waves per SIMD with the log, four with atomics (kWavesPerEuLoggedAdjoint)
+        if constexpr (kTapeAdjoint<F>)
+          go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
+        else if (log.param >= 0)
+          go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint>);
+        else
+          go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
+      });
+    reduce_log(s, GL, stream, log);
+  }
   else if (d->type == RCV_INTEGRATOR_VOLPATH)
     with_render_features(s->features(), [&](auto f) {
       hipLaunchKernelGGL((adjoint_kernel<RCV_INTEGRATOR_VOLPATH, decltype(f)::value>), dim3(grid), dim3(block),
@@ -1006,7 +1058,15 @@ int launch_forward(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
   const int block = d->block_size ? d->block_size : kDefaultBlock;
   const unsigned grid = ceil_div(n_pix << cl2, block);
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
-  if (d->type == RCV_INTEGRATOR_VOLPATH)
+  if (takes_box(s, d)) {
+    const int ucl2 = box_chunk_log2(s, n_pix, spp, cl2, 3);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    launch_box(s, 1, kBoxForward,
+               BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), nullptr, &T, s->partial,
+                         s->work_queue});
+    hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+                       ucl2, spp, nullptr, dimg);
+  } else if (d->type == RCV_INTEGRATOR_VOLPATH)
     with_render_features(s->features(), [&](auto f) {
       hipLaunchKernelGGL((forward_kernel<RCV_INTEGRATOR_VOLPATH, decltype(f)::value>), dim3(grid), dim3(block),
                          stack_bytes(block), stream, s->view, I, sensor, seed, spp, spt, cl2, T, dimg);

@@ -80,6 +80,41 @@ __host__ __device__ inline int sample_end(int c, int spp, int chunk_log2) {
   return int((int64_t(c + 1) * spp) >> chunk_log2);
 }
 
+// Render, adjoint and forward mode of the one-box volume tracker.
+constexpr int kBoxRender = 0;
+constexpr int kBoxAdjoint = 1;
+constexpr int kBoxForward = 2;
+
+// Waves per SIMD of the one-box volume tracker (boxpath.hpp): four, up to 128
+// VGPRs. It is bound by instruction issue; three and five waves measured
+// within 3 % of four.
+template <int NS, int MODE>
+constexpr int kBoxWaves = 4;
+
+// Blocks of `kern` the current device holds at once (compute units x
+// resident blocks per unit) with `lds` bytes of dynamic LDS per block,
+// cached per (device, kernel, block size).
+unsigned resident_grid(const void *kern, int block, size_t lds);
+
+struct GradTargets;
+
+// One launch of the one-box volume tracker (box.hip): work units, where the
+// unit sums go (render, forward) and the gradients or tangents.
+struct BoxLaunch {
+  hipStream_t stream;
+  int block;
+  IntegArgs I;
+  int sensor;
+  uint32_t seed;
+  int spp, chunk_log2;
+  unsigned units;
+  const float *grad_img;
+  const GradTargets *G;
+  float *partial;
+  unsigned *queue;
+};
+void launch_box(const Scene *s, int ns, int mode, const BoxLaunch &L);
+
 int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint32_t seed, int spp,
                   float *img_old, float *img_new, int ns, hipStream_t stream, const char *fn);
 

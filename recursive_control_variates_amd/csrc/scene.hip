@@ -371,7 +371,7 @@ int Scene::upload(hipStream_t stream) {
   {
     int64_t max_pix = 0;
     for (auto &sen : sensors) max_pix = std::max(max_pix, int64_t(sen.film_w) * sen.film_h);
-    partial_cap = max_pix * kRenderMaxUnitsPerPixel * 6;
+    partial_cap = std::max(max_pix * kRenderMaxUnitsPerPixel, std::min(max_pix * 64, kRenderMinUnits)) * 6;
     if (partial_cap > 0)
       RCV_TRY_HIP(hipMalloc(&partial, size_t(partial_cap) * sizeof(float)), "rcv_scene_commit: hipMalloc");
   }
@@ -436,6 +436,20 @@ int Scene::upload(hipStream_t stream) {
     }
   }
   n_nodes = int(b.nodes.size());
+  one_box = shapes.size() == 1 && box_shape.size() == 1 && tri_shape.empty() && sph_shape.empty() &&
+            media.size() == 1 && !media[0].homogeneous && media[0].sample_emitters && shapes[0].interior == 0 &&
+            shapes[0].exterior == -1 && shapes[0].emitter < 0 && shapes[0].bsdf >= 0 &&
+            bsdfs[shapes[0].bsdf].type == RCV_BSDF_NULL && emitters.size() == 1 &&
+            emitters[0].type == RCV_EMITTER_CONSTANT;
+  if (one_box) {
+    box_scene.root = b.nodes[0];
+    box_scene.box = boxes[0];
+    for (int k = 0; k < 3; ++k) {
+      box_scene.env[k] = emitters[0].rgb[k];
+      box_scene.bs_center[k] = bs_center[k];
+    }
+    box_scene.bs_radius = bs_radius;
+  }
   if (int rc = alloc_supergrids()) return rc;
   committed = true;
   // Majorants of states bound before commit.
@@ -542,6 +556,17 @@ int Scene::features() const {
     if (m.supergrid_offset >= 0) f |= kFeatSupergrid;
   }
   return f;
+}
+
+// The tracker's lookups read pairs of neighbours along x with 32-bit byte
+// offsets and form indices with 24-bit multiplies: rows of at least two
+// voxels, fewer than 2^29 voxels in fewer than 2^24 rows. Launches that count
+// events take the general kernels.
+bool Scene::box_path() const {
+  if (!one_box || view.counters) return false;
+  const Param &p = params[media[0].sigma_param];
+  return p.nx >= 2 && p.nx < (1 << 24) && int64_t(p.ny) * p.nz < (int64_t(1) << 24) &&
+         int64_t(p.nx) * p.ny * p.nz < (int64_t(1) << 29);
 }
 
 Scene::~Scene() {

@@ -15,6 +15,9 @@ namespace rcv {
 // state of the optimisation 15.9 / 21.5 -> 12.6 / 15.8 ms, 3.1 -> 3.7 ms at
 // the uniform initial state (eight: 12.3 / 14.8, 4.4 ms).
 constexpr int kRenderMaxUnitsPerPixel = 4;
+// Small images may be split further, into up to 64 units per pixel, as long
+// as the buffer stays within this many units (25 MB).
+constexpr int64_t kRenderMinUnits = int64_t(1) << 20;
 
 struct Param {
   int kind = 0;
@@ -55,6 +58,8 @@ struct Scene {
   float bs_center[3] = {0, 0, 0};
   float bs_radius = 0;
   SceneView view{};
+  bool one_box = false;             // box_scene describes the scene (set at commit)
+  BoxScene box_scene{};
 
   Scene() = default;
   Scene(const Scene &) = delete;
@@ -68,6 +73,7 @@ struct Scene {
   int alloc_supergrids();
   int relayout_supergrids(hipStream_t stream);
   int features() const;  // kFeat* mask of the committed scene
+  bool box_path() const;  // whether the one-box volume tracker covers the scene
 };
 
 // Decodes an order-preserving key written by the majorant reduction.

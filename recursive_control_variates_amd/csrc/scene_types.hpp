@@ -162,4 +162,25 @@ struct SceneView {
   ParamBind params[kMaxParams];
 };
 
+struct IntegArgs {
+  int max_depth;
+  int rr_depth;
+  int hide_emitters;
+  int flags;  // integrator-specific switches (volpathsimple: kSimpleNo*)
+};
+
+// A scene of one heterogeneous medium (interior of one box with a null BSDF,
+// nothing outside) under a constant environment, by value in the kernel
+// arguments.
+struct BoxScene {
+  MediumInfo med;
+  ParamBind sigma, albedo;  // albedo unused for a constant albedo
+  BVHNode root;             // the scene's BVH: one leaf holding the box
+  BoxPrim box;
+  float env[3];
+  float bs_center[3];
+  float bs_radius;
+  int32_t unit_extent;      // med.hi - med.lo == 1 on every axis: x / 1 is x
+};
+
 }  // namespace rcv

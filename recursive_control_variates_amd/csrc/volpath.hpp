@@ -23,13 +23,6 @@
 
 namespace rcv {
 
-struct IntegArgs {
-  int max_depth;
-  int rr_depth;
-  int hide_emitters;
-  int flags;  // integrator-specific switches (volpathsimple: kSimpleNo*)
-};
-
 // Scatter log geometry: reduction tiles of a logged gradient, bins (one per
 // tile, then one per seam between tiles t and t + 1), records per chunk.
 constexpr int kLogMaxTiles = 16;
