@@ -32,10 +32,8 @@
 #include <cstring>
 #include <vector>
 
-#include "common.hpp"
+#include "batch_internal.hpp"
 #include "path.hpp"
-#include "render_internal.hpp"
-#include "volpath.hpp"
 
 namespace rcv {
 
@@ -44,68 +42,11 @@ constexpr int kElemBlock = 256;
 constexpr int kBatchMaxSpt = 32;         // camera samples per work unit (at most)
 constexpr int64_t kBatchMinThreads = 0;  // the batch, not one job, fills the device
 
-struct BatchJobDev {
-  SceneView view;       // params[param].data[] rotated on the device
-  IntegArgs integ;
-  int32_t itype;        // RCV_INTEGRATOR_*
-  int32_t method;       // 0 baseline (plain), 1 cv_ps (two-state + combine)
-  int32_t loss;         // RCV_LOSS_*
-  int32_t sensor;
-  int32_t spp, spt, cl2;
-  int32_t spp_g, spt_g, cl2_g;
-  int32_t film_w, n_pix;
-  uint32_t seed;
-  int32_t param;
-  int64_t n_param;
-  int64_t n_img;
-  int64_t unit_begin, unit_begin_g;  // in this job's render / adjoint class space
-  int64_t elem_begin, pelem_begin;   // padded image / parameter element offsets
-  float *ring[3];
-  int32_t ring_old, ring_new, ring_next;
-  uint32_t *maj_keys;   // scene majorant keys of `param`: [OLD], [NEW]
-  uint32_t next_key;    // max key of the ring's next buffer (written by adam)
-  int32_t iter;
-  int32_t active;       // 0: the job sits out this iteration (no state changes)
-  float *H, *F, *img, *grad_img;
-  const float *img_ref;
-  float *cv[8];
-  int32_t warmup;
-  float cv_b1, cv_b2;
-  double cv_log_b1, cv_log_b2;
-  int32_t pre_update;
-  float *grad, *m, *v;
-  GradTargets gt;       // gt.g[param] = grad, others null
-  float lr, b1, b2, eps, clamp_lo, clamp_hi;
-  double log_b1, log_b2;
-  float *sg_out;        // supergrids [OLD][NEW] of the optimised grid's medium, or null
-  int32_t sg_res[3];
-};
-
 namespace {
-
-__device__ inline int find_job(const int64_t *__restrict__ ends, int n, int64_t u) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (ends[mid] <= u)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
 
 __device__ inline uint32_t float_key_dev(float f) {
   const uint32_t u = __builtin_bit_cast(uint32_t, f);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
-__device__ inline uint32_t iter_seed(const BatchJobDev &J) { return J.seed + uint32_t(J.iter); }
-
-__device__ inline uint32_t iter_seed_grad(const BatchJobDev &J) {
-  uint32_t a = iter_seed(J), b = 1u;
-  tea(a, b);
-  return a;
 }
 
 // ---------------------------------------------------------------- 1. rotate
@@ -114,6 +55,7 @@ __global__ void batch_rotate_kernel(BatchJobDev *jobs, int n_jobs, unsigned *que
   if (j < 6) queues[j] = 0u;
   if (j >= n_jobs) return;
   BatchJobDev &J = jobs[j];
+  if (J.box_queue) J.box_queue[0] = J.box_queue[1] = 0u;
   if (!J.active) return;
   if (J.iter > 0) {
     const int old_slot = J.ring_old;
@@ -124,6 +66,10 @@ __global__ void batch_rotate_kernel(BatchJobDev *jobs, int n_jobs, unsigned *que
     J.view.params[J.param].data[RCV_STATE_NEW] = J.ring[J.ring_new];
     J.maj_keys[RCV_STATE_OLD] = J.maj_keys[RCV_STATE_NEW];
     J.maj_keys[RCV_STATE_NEW] = J.next_key;
+    if (J.box_queue) {
+      J.box.sigma = J.view.params[J.box.med.sigma_param];
+      if (J.box.med.albedo_param >= 0) J.box.albedo = J.view.params[J.box.med.albedo_param];
+    }
   }
   J.next_key = float_key_dev(-kInf);
 }
@@ -215,6 +161,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
   }
 }
 
+// Image element i of a one-box job from its unit sums, units in order
+// (reduce_units_kernel).
+__device__ inline void unit_means(const BatchJobDev &J, int64_t i) {
+  const int64_t pixel = i / 3;
+  const int ns = J.method == 1 ? 2 : 1, c = int(i - 3 * pixel);
+  const int units = 1 << J.box_cl2;
+  const float *src = J.box_partial + (pixel << J.box_cl2) * (3 * ns) + c;
+  for (int k = 0; k < ns; ++k) {
+    float x = src[3 * k];
+    for (int q = 1; q < units; ++q) x += src[q * (3 * ns) + 3 * k];
+    (k == ns - 1 ? J.F : J.H)[i] = x / float(J.spp);
+  }
+}
+
 // ----------------------------------------------- 3+4. combine, loss gradient
 // One block of 256 elements belongs to one job (element ranges are padded).
 __global__ __launch_bounds__(kElemBlock) void batch_combine_loss_kernel(BatchJobDev *__restrict__ jobs,
@@ -227,6 +187,7 @@ __global__ __launch_bounds__(kElemBlock) void batch_combine_loss_kernel(BatchJob
   if (!J.active) return;
   const int64_t i = e0 + threadIdx.x - J.elem_begin;
   if (i >= J.n_img) return;
+  if (J.box_partial) unit_means(J, i);
   const float f = J.F[i];
   float out;
   if (J.method == 1) {
@@ -398,6 +359,14 @@ struct BatchClass {
 struct Batch {
   std::vector<BatchJobDev> host_jobs;
   std::vector<const Scene *> scenes;
+  std::vector<char> is_box;  // jobs that take the one-box tracker
+  // the one-box adjoints' scatter log: its pool (null: none), the logged
+  // gradients (first of them, table on the device), tiles in all
+  LogBuf log;
+  GradTargets pool;
+  std::vector<LogTarget> log_targets;
+  LogTarget *d_log_targets = nullptr;
+  int log_tiles = 0, device = 0;
   bool committed = false;
   void *dev = nullptr;
   BatchJobDev *d_jobs = nullptr;
@@ -406,6 +375,11 @@ struct Batch {
   unsigned *d_queues = nullptr;
   BatchClass render_cls[4];  // (itype, ns): 0 path/1, 1 path/2, 2 vol/1, 3 vol/2
   BatchClass adj_cls[2];     // itype
+  // one-box volume jobs by feature mask (albedo grid, supergrid): renders of
+  // one and two states, adjoints
+  BatchClass box_cls[4][3];
+  int32_t *d_box_ids[4][3] = {};
+  int64_t *d_box_ends[4][3] = {};
   int32_t *d_ids[6] = {nullptr};
   int64_t *d_ends[6] = {nullptr};
   std::vector<int32_t> sg_ids;   // jobs whose optimised grid has a supergrid
@@ -420,7 +394,8 @@ struct Batch {
     for (const Scene *s : scenes) --const_cast<Scene *>(s)->batch_refs;
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (dev) (void)hipFree(dev);
+    if (dev) (void)hipFree(dev);  // waits for the batch's launches
+    if (log.rec) give_log_pool(log, device);
   }
 };
 
@@ -534,12 +509,32 @@ extern "C" int rcv_batch_add_job(rcv_batch *b, const rcv_batch_job *d, int32_t *
     }
   RCV_REQUIRE(n_sg <= 1, "rcv_batch_add_job: the optimised grid drives %d media with supergrids (at most 1)", n_sg);
   RCV_REQUIRE(!(s->features() & kFeatHomog), "rcv_batch_add_job: batched jobs take heterogeneous media only");
-  if (J.itype == RCV_INTEGRATOR_VOLPATH) b->feat |= s->features();
+  // the one-box tracker takes a volume job as a single launch's (an explicit
+  // samples_per_thread asks for the general kernels)
+  J.box_queue = nullptr;
+  J.box_partial = nullptr;
+  const bool box = takes_box(s, &d->integrator);
+  if (box) J.box = bound_box(s);
+  b->is_box.push_back(box);
+  if (J.itype == RCV_INTEGRATOR_VOLPATH && !box) b->feat |= s->features();
   b->host_jobs.push_back(J);
   b->scenes.push_back(s);
   ++const_cast<Scene *>(s)->batch_refs;
   if (out_job) *out_job = int(b->host_jobs.size()) - 1;
   return RCV_OK;
+}
+
+// Work units per pixel (log2) of a one-box job: the adjoint's units trace
+// kVolUnitSamples samples; the renders' at least 8, so that their unit sums
+// (24 bytes per unit) stay small beside the images, or kVolUnitSamples in a
+// batch of few pixels, whose launches wait for their longest unit (12 jobs of
+// 80 to 160 pixels a side, 6 to 12 samples: the render 3.9 -> 1.9 ms).
+constexpr int64_t kFewPixels = int64_t(1) << 19;
+static int batch_box_chunk_log2(int spp, bool adjoint, int64_t batch_pixels) {
+  const int least = adjoint || batch_pixels <= kFewPixels ? kVolUnitSamples : 8;
+  int cl2 = 0;
+  while (cl2 < 6 && (spp >> (cl2 + 1)) >= least) ++cl2;
+  return cl2;
 }
 
 static int64_t pad(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -550,7 +545,9 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
   const int n = int(b->host_jobs.size());
   RCV_REQUIRE(n > 0 && n <= RCV_BATCH_MAX_JOBS, "rcv_batch_commit: 1..%d jobs", RCV_BATCH_MAX_JOBS);
   std::vector<int64_t> elem_ends(n), pelem_ends(n);
-  int64_t e = 0, pe = 0;
+  int64_t e = 0, pe = 0, partial_floats = 0, batch_pixels = 0;
+  for (int j = 0; j < n; ++j)
+    if (b->is_box[j]) batch_pixels += b->host_jobs[j].n_pix;
   for (int j = 0; j < n; ++j) {
     BatchJobDev &J = b->host_jobs[j];
     J.elem_begin = e;
@@ -559,6 +556,19 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     J.pelem_begin = pe;
     pe += pad(J.n_param, kElemBlock);
     pelem_ends[j] = pe;
+    if (b->is_box[j]) {
+      const int f = (b->scenes[j]->features() & (kFeatAlbedoGrid | kFeatSupergrid)) / kFeatAlbedoGrid;
+      for (int a = 0; a < 2; ++a) {
+        BatchClass &c = b->box_cls[f][a == 1 ? 2 : (J.method == 1 ? 1 : 0)];
+        const int cl2 = batch_box_chunk_log2(a == 1 ? J.spp_g : J.spp, a == 1, batch_pixels);
+        (a == 1 ? J.box_cl2_g : J.box_cl2) = cl2;
+        c.total += int64_t(J.n_pix) << cl2;
+        c.ids.push_back(j);
+        c.ends.push_back(c.total);
+      }
+      if (J.box_cl2 > 0) partial_floats += (int64_t(J.n_pix) << J.box_cl2) * 3 * (J.method == 1 ? 2 : 1);
+      continue;
+    }
     const int rc_i = (J.itype == RCV_INTEGRATOR_VOLPATH ? 2 : 0) + (J.method == 1 ? 1 : 0);
     BatchClass &rc = b->render_cls[rc_i];
     J.unit_begin = rc.total;
@@ -575,6 +585,7 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     RCV_REQUIRE(c.total < (int64_t(1) << 31), "rcv_batch_commit: too many work units");
   for (auto &c : b->adj_cls)
     RCV_REQUIRE(c.total < (int64_t(1) << 31), "rcv_batch_commit: too many work units");
+  // (a job's own units fit 32 bits: pixels * spp do)
   b->elem_total = e;
   b->pelem_total = pe;
   b->sg_ids.clear();
@@ -586,6 +597,23 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     sg_total += 2 * int64_t(J.sg_res[0]) * J.sg_res[1] * J.sg_res[2];
     b->sg_ids.push_back(j);
     b->sg_ends.push_back(sg_total);
+  }
+  // the scatter log of the one-box jobs whose density gradient fits it
+  b->pool.clear();
+  (void)hipGetDevice(&b->device);
+  for (int j = 0; j < n; ++j) {
+    BatchJobDev &J = b->host_jobs[j];
+    if (!b->is_box[j] || J.box.med.sigma_param != J.param) continue;
+    LogTarget t;
+    const int tiles = log_target(b->scenes[j], J.box.med, J.grad, t);
+    if (tiles == 0) continue;
+    if (!b->log.rec && !take_log_pool(b->log)) break;  // without memory: atomics
+    t.bin0 = unsigned(kLogBins * b->log_targets.size());
+    t.tile0 = b->log_tiles;
+    log_into(b->log, J.param, t.bin0, J.gt);
+    log_into(b->log, -1, 0, b->pool);
+    b->log_tiles += tiles;
+    b->log_targets.push_back(t);
   }
   // device block: jobs | elem ends | pelem ends | queues | class ids/ends
   size_t bytes = 0;
@@ -606,9 +634,29 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     o_ids[c] = reserve(4 * bc.ids.size());
     o_ends[c] = reserve(8 * bc.ends.size());
   }
+  size_t o_bids[4][3], o_bends[4][3];
+  for (int f = 0; f < 4; ++f)
+    for (int k = 0; k < 3; ++k) {
+      o_bids[f][k] = reserve(4 * b->box_cls[f][k].ids.size());
+      o_bends[f][k] = reserve(8 * b->box_cls[f][k].ends.size());
+    }
+  const size_t o_log = reserve(sizeof(LogTarget) * b->log_targets.size());
+  const size_t o_bq = reserve(2 * sizeof(unsigned) * n);
+  const size_t uploaded = bytes;
+  const size_t o_part = reserve(4 * size_t(partial_floats));
   RCV_TRY_HIP(hipMalloc(&b->dev, bytes), "rcv_batch_commit: hipMalloc");
   char *base = static_cast<char *>(b->dev);
-  std::vector<char> blob(bytes, 0);
+  float *part = reinterpret_cast<float *>(base + o_part);
+  for (int j = 0; j < n; ++j) {
+    BatchJobDev &J = b->host_jobs[j];
+    if (!b->is_box[j]) continue;
+    J.box_queue = reinterpret_cast<unsigned *>(base + o_bq) + 2 * j;
+    if (J.box_cl2 > 0) {
+      J.box_partial = part;
+      part += (int64_t(J.n_pix) << J.box_cl2) * 3 * (J.method == 1 ? 2 : 1);
+    }
+  }
+  std::vector<char> blob(uploaded, 0);
   std::memcpy(blob.data() + o_jobs, b->host_jobs.data(), sizeof(BatchJobDev) * n);
   std::memcpy(blob.data() + o_ee, elem_ends.data(), 8 * n);
   std::memcpy(blob.data() + o_pe, pelem_ends.data(), 8 * n);
@@ -627,8 +675,21 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     b->d_ids[c] = reinterpret_cast<int32_t *>(base + o_ids[c]);
     b->d_ends[c] = reinterpret_cast<int64_t *>(base + o_ends[c]);
   }
+  for (int f = 0; f < 4; ++f)
+    for (int k = 0; k < 3; ++k) {
+      const BatchClass &bc = b->box_cls[f][k];
+      if (!bc.ids.empty()) {
+        std::memcpy(blob.data() + o_bids[f][k], bc.ids.data(), 4 * bc.ids.size());
+        std::memcpy(blob.data() + o_bends[f][k], bc.ends.data(), 8 * bc.ends.size());
+      }
+      b->d_box_ids[f][k] = reinterpret_cast<int32_t *>(base + o_bids[f][k]);
+      b->d_box_ends[f][k] = reinterpret_cast<int64_t *>(base + o_bends[f][k]);
+    }
+  if (!b->log_targets.empty())
+    std::memcpy(blob.data() + o_log, b->log_targets.data(), sizeof(LogTarget) * b->log_targets.size());
+  b->d_log_targets = reinterpret_cast<LogTarget *>(base + o_log);
   hipStream_t st = as_stream(stream);
-  RCV_TRY_HIP(hipMemcpyAsync(b->dev, blob.data(), bytes, hipMemcpyHostToDevice, st), "rcv_batch_commit: upload");
+  RCV_TRY_HIP(hipMemcpyAsync(b->dev, blob.data(), uploaded, hipMemcpyHostToDevice, st), "rcv_batch_commit: upload");
   RCV_TRY_HIP(hipStreamSynchronize(st), "rcv_batch_commit: synchronize");
   b->d_jobs = reinterpret_cast<BatchJobDev *>(base + o_jobs);
   b->d_elem_ends = reinterpret_cast<int64_t *>(base + o_ee);
@@ -721,6 +782,14 @@ static int enqueue_step(rcv_batch *b, hipStream_t st) {
       });
     if (int rc = check_launch("rcv_batch_step: render")) return rc;
   }
+  for (int f = 0; f < 4; ++f)
+    for (int k = 0; k < 2; ++k) {
+      const BatchClass &bc = b->box_cls[f][k];
+      if (bc.total == 0) continue;
+      launch_box_batch(f * kFeatAlbedoGrid, k + 1, b->d_jobs,
+                       BoxClass{b->d_box_ids[f][k], b->d_box_ends[f][k], int(bc.ids.size())}, bc.total, b->block, b->pool, st);
+      if (int rc = check_launch("rcv_batch_step: render")) return rc;
+    }
   hipLaunchKernelGGL(batch_combine_loss_kernel, dim3(unsigned(b->elem_total / kElemBlock)), dim3(kElemBlock), 0,
                      st, b->d_jobs, b->d_elem_ends, n);
   hipLaunchKernelGGL(batch_zero_grad_kernel, dim3(unsigned(b->pelem_total / kElemBlock)), dim3(kElemBlock), 0, st,
@@ -742,6 +811,16 @@ static int enqueue_step(rcv_batch *b, hipStream_t st) {
       });
     if (int rc = check_launch("rcv_batch_step: adjoint")) return rc;
   }
+  if (b->log.rec) zero_log(b->log, st);
+  for (int f = 0; f < 4; ++f) {
+    const BatchClass &bc = b->box_cls[f][2];
+    if (bc.total == 0) continue;
+    launch_box_batch(f * kFeatAlbedoGrid, 0, b->d_jobs,
+                     BoxClass{b->d_box_ids[f][2], b->d_box_ends[f][2], int(bc.ids.size())}, bc.total, b->block, b->pool, st);
+    if (int rc = check_launch("rcv_batch_step: adjoint")) return rc;
+  }
+  if (b->log.rec)
+    reduce_log_batch(b->log, b->log_targets[0], b->d_log_targets, int(b->log_targets.size()), b->log_tiles, st);
   hipLaunchKernelGGL(batch_adam_kernel, dim3(unsigned(b->pelem_total / kElemBlock)), dim3(kElemBlock), 0, st,
                      b->d_jobs, b->d_pelem_ends, n);
   hipLaunchKernelGGL(batch_advance_kernel, dim3(ceil_div(n, 64)), dim3(64), 0, st, b->d_jobs, n);

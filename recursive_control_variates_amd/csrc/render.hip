@@ -22,6 +22,7 @@
 #include "common.hpp"
 #include "path.hpp"
 #include "render_internal.hpp"
+#include "scatter_log.hpp"
 #include "volpath.hpp"
 #include "volsimple.hpp"
 
@@ -31,14 +32,6 @@ namespace {
 constexpr int kMaxBlock = 256;      // launch bound of the render kernels
 constexpr int kDefaultBlock = 256;  // threads per block when the descriptor says 0
 constexpr int kAdjUnitSamples = 16;  // camera samples per work unit of the persistent per-sample adjoints
-// Camera samples per work unit of the volume path tracer's persistent
-// launches (the adjoint; the renders, within kRenderMaxUnitsPerPixel). With
-// small units the lanes of a wavefront trace samples of the same few pixels,
-// whose paths start alike and share L1 lines of the grid, and the last units
-// of a launch are short. The 64^3 adjoint at the mid / final state of the
-// optimisation: 46.1 / 67.5 ms with 16-sample units, 39.7 / 51.4 with 8,
-// 37.0 / 47.8 with 4, 36.2 / 46.4 with 2.
-constexpr int kVolUnitSamples = 2;
 
 template <int NS, int INTEG, int F>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(kWavesPerEuRender<NS, INTEG>))) void render_kernel(
@@ -277,154 +270,8 @@ adjoint_persistent_kernel(SceneView S, IntegArgs I, int sensor, uint32_t seed, i
   }
   if constexpr ((F & kFeatHomog) != 0) flush_homogeneous(S, G, t.hom);
   // the whole wavefront is past its loop
+  log_close(G, stack);
   log_end(G, stack);
-}
-
-// Scatter log reduction. Block (x, y) takes tile y of the gradient
-// (voxels [y tile, (y + 1) tile)) and its share of the chunks of the three
-// bins whose records reach into it (tile y, the seams below and above it);
-// a record is read once, or twice when it lies across a seam. A block of
-// kReduceBlock threads takes kStepChunks chunks per step: thread i reads
-// slot i % kLogChunk of kReduceUnroll of them, all loads in flight together
-// (unused slots are read, every index stays inside the pool, and skipped).
-// The records of one chunk come from one wavefront of the adjoint, whose
-// lanes trace neighbouring pixels; the 8-lane groups of a wavefront take
-// their chunks in rotated order so that one instruction adds records of
-// several chunks.
-constexpr int kReduceBlock = 1024;
-constexpr int kReduceUnroll = 8;
-constexpr unsigned kChunkGroups = unsigned(kReduceBlock) / kLogChunk;
-constexpr unsigned kStepChunks = kChunkGroups * kReduceUnroll;
-static_assert(kReduceBlock % int(kLogChunk) == 0, "a reduction block covers whole chunks");
-
-// Calls fn(record) for each record of the block's share.
-template <class Fn>
-__device__ inline void log_block_records(const int4 *__restrict__ rec, const unsigned *__restrict__ ctl,
-                                         const unsigned *__restrict__ list,
-                                         const unsigned *__restrict__ fill, unsigned nchunks, Fn &&fn) {
-  const int y = int(blockIdx.y);
-  const unsigned slot = threadIdx.x % kLogChunk;
-  const unsigned sub = threadIdx.x / kLogChunk;
-  const unsigned grp = (threadIdx.x >> 3) % kReduceUnroll;
-  for (int k = 0; k < 3; ++k) {
-    if (k == 1 && y == 0) continue;
-    const int b = k == 0 ? y : kLogMaxTiles + y - (k == 1 ? 1 : 0);
-    const unsigned nb = min(ctl[1 + b], nchunks);
-    const unsigned *bl = list + size_t(b) * nchunks;
-    for (unsigned p0 = blockIdx.x * kStepChunks; p0 < nb; p0 += gridDim.x * kStepChunks) {
-      unsigned c[kReduceUnroll], n[kReduceUnroll];
-      int4 e[kReduceUnroll];
-#pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u) {
-        const unsigned j = p0 + sub + kChunkGroups * ((grp + unsigned(u)) % kReduceUnroll);
-        c[u] = j < nb ? bl[j] : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u) {
-        const unsigned j = p0 + sub + kChunkGroups * ((grp + unsigned(u)) % kReduceUnroll);
-        n[u] = j < nb ? min(fill[c[u]], kLogChunk) : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u) e[u] = rec[size_t(c[u]) * kLogChunk + slot];
-#pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u)
-        if (slot < n[u]) fn(e[u]);
-    }
-  }
-}
-
-// Calls add(voxel - lo, value x weight) for the corners of a record
-// (log_record) that fall in [lo, hi): the products of scatter_grid, with
-// the fractions as stored.
-template <class Add>
-__device__ inline void record_corners(const int4 &e, int nx, int nxy, int64_t lo, int64_t hi, Add &&add) {
-  const unsigned cell = unsigned(e.x);
-  const unsigned long long q = (unsigned long long)unsigned(e.y) | ((unsigned long long)unsigned(e.z) << 32);
-  constexpr unsigned kMask = (1u << 21) - 1u;
-  GridFoot f;
-  f.base = int(cell & kRecBaseMask);
-  f.dx = int((cell >> 26) & 1u);
-  f.dy = ((cell >> 27) & 1u) ? nx : 0;
-  f.dz = ((cell >> 28) & 1u) ? nxy : 0;
-  f.tx = float(unsigned(q) & kMask) / kLogFracScale;
-  f.ty = float(unsigned(q >> 21) & kMask) / kLogFracScale;
-  f.tz = float(unsigned(q >> 42) & kMask) / kLogFracScale;
-  const float x = __int_as_float(e.w);
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int64_t idx = f.idx(q);
-    if (idx >= lo && idx < hi) add(idx - lo, x * f.w(q));
-  }
-}
-
-// Adds the scatter log of a persistent adjoint launch to the gradient of
-// an nx x ny x nz grid, tile by tile (see log_block_records). The tile is
-// summed in LDS in 64-bit fixed point: integer LDS atomics run ~5x faster
-// than float ones here. A first pass over the share's values finds its
-// record count N and largest magnitude M; terms are scaled by 2^s with M N
-// 2^s <= 2^62, so no partial sum overflows and each term is kept to ~2^-44
-// of M (float atomics keep 2^-24 of the running sum). A share holding a
-// non-finite value is summed with float atomics as it stands.
-__global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const int4 *__restrict__ rec,
-                                                              const unsigned *__restrict__ ctl,
-                                                              const unsigned *__restrict__ list,
-                                                              const unsigned *__restrict__ fill, unsigned nchunks,
-                                                              int nx, int nxy, int64_t nvox, int tile,
-                                                              float *__restrict__ g) {
-  extern __shared__ long long acc[];  // tile words (floats in the first half for a non-finite share)
-  __shared__ float wave_max[kReduceBlock / 64];
-  __shared__ unsigned wave_count[kReduceBlock / 64];
-  const int64_t lo = int64_t(blockIdx.y) * tile;
-  const int64_t hi = min(lo + int64_t(tile), nvox);
-  float m = 0.0f;
-  unsigned total = 0;
-  log_block_records(rec, ctl, list, fill, nchunks, [&](const int4 &e) {
-    const float a = fabsf(__int_as_float(e.w));
-    m = (a <= m) ? m : (a == a ? a : INFINITY);  // NaN and inf both give inf
-    ++total;
-  });
-  for (int off = 32; off > 0; off >>= 1) {
-    m = fmaxf(m, __shfl_xor(m, off, 64));
-    total += __shfl_xor(total, off, 64);
-  }
-  if ((threadIdx.x & 63u) == 0) {
-    wave_max[threadIdx.x >> 6] = m;
-    wave_count[threadIdx.x >> 6] = total;
-  }
-  __syncthreads();
-  m = 0.0f;
-  total = 0;
-  for (int w = 0; w < kReduceBlock / 64; ++w) {
-    m = fmaxf(m, wave_max[w]);
-    total += wave_count[w];
-  }
-  if (total == 0 || m == 0.0f) return;
-  if (isfinite(m)) {
-    int em = 0, en = 0;
-    (void)frexpf(m, &em);               // m < 2^em
-    (void)frexpf(float(total), &en);    // total <= 2^en
-    const int sc = 62 - em - en;
-    for (int v = threadIdx.x; v < tile; v += blockDim.x) acc[v] = 0;
-    __syncthreads();
-    log_block_records(rec, ctl, list, fill, nchunks, [&](const int4 &e) {
-      record_corners(e, nx, nxy, lo, hi, [&](int64_t a, float t) {
-        atomicAdd(reinterpret_cast<unsigned long long *>(&acc[a]), (unsigned long long)__float2ll_rn(ldexpf(t, sc)));
-      });
-    });
-    __syncthreads();
-    for (int64_t v = threadIdx.x; v < hi - lo; v += blockDim.x)
-      if (acc[v] != 0) atomicAdd(&g[lo + v], ldexpf(__ll2float_rn(acc[v]), -sc));
-  } else {
-    float *facc = reinterpret_cast<float *>(acc);
-    for (int v = threadIdx.x; v < tile; v += blockDim.x) facc[v] = 0.0f;
-    __syncthreads();
-    log_block_records(rec, ctl, list, fill, nchunks, [&](const int4 &e) {
-      record_corners(e, nx, nxy, lo, hi, [&](int64_t a, float t) { atomicAdd(&facc[a], t); });
-    });
-    __syncthreads();
-    for (int64_t v = threadIdx.x; v < hi - lo; v += blockDim.x)
-      if (facc[v] != 0.0f) atomicAdd(&g[lo + v], facc[v]);
-  }
 }
 
 // The per-sample integrators' adjoint (volpathsimple, surface path tracer) as
@@ -590,94 +437,6 @@ unsigned resident_grid(const void *kern, int block, size_t lds) {
   const unsigned g = unsigned(std::max(1, per_cu) * std::max(1, cus));
   cache[key] = g;
   return g;
-}
-
-// Scatter log of the persistent volume adjoint: a pool of kLogPool chunks
-// of kLogChunk 16-byte records (3.2 GB, and 100 MB of chunk lists), one per
-// (device, stream), kept for the process (launches on one stream run in
-// order; other streams get their own). The reduction tiles hold up to
-// 16384 voxels (128 KB of LDS, less where the device allows less); grids of
-// more than kLogMaxTiles tiles, or whose footprints span more than two
-// tiles, keep the atomics. kLogSplits blocks share each tile's reduction.
-constexpr unsigned kLogPool = 786432;
-constexpr int kLogSplits = 64;
-
-struct LogBuf {
-  int4 *rec = nullptr;
-  unsigned *ctl = nullptr;   // 1 + kLogBins counters
-  unsigned *list = nullptr;  // kLogBins x kLogPool chunk indices
-  unsigned *fill = nullptr;  // kLogPool record counts
-};
-
-static int log_buffer(hipStream_t stream, LogBuf &out) {
-  static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, LogBuf> bufs;
-  int dev = 0;
-  RCV_TRY_HIP(hipGetDevice(&dev), "hipGetDevice");
-  std::lock_guard<std::mutex> lock(mu);
-  const auto key = std::make_pair(dev, stream);
-  auto it = bufs.find(key);
-  if (it == bufs.end()) {
-    LogBuf nb;
-    const size_t recs = size_t(kLogPool) * kLogChunk;
-    hipError_t e = hipMalloc(&nb.rec, recs * sizeof(int4));
-    if (e == hipSuccess) e = hipMalloc(&nb.ctl, (1 + kLogBins) * sizeof(unsigned));
-    if (e == hipSuccess) e = hipMalloc(&nb.list, size_t(kLogBins) * kLogPool * sizeof(unsigned));
-    if (e == hipSuccess) e = hipMalloc(&nb.fill, size_t(kLogPool) * sizeof(unsigned));
-    if (e != hipSuccess) {
-      (void)hipFree(nb.rec);
-      (void)hipFree(nb.ctl);
-      (void)hipFree(nb.list);
-      (void)hipFree(nb.fill);
-      return hip_fail(e, "scatter log: allocation");
-    }
-    it = bufs.emplace(key, nb).first;
-  }
-  out = it->second;
-  return RCV_OK;
-}
-
-// Chunks of the pool a launch may draw: kLogPool, or fewer when the
-// environment sets RCV_SCATTER_LOG_CHUNKS (a test of the adjoint past the
-// pool's end, where the scatter-adds fall back to atomics).
-static unsigned log_pool_chunks() {
-  const char *e = std::getenv("RCV_SCATTER_LOG_CHUNKS");
-  if (!e || !*e) return kLogPool;
-  char *end = nullptr;
-  const unsigned long v = std::strtoul(e, &end, 10);
-  if (end == e || *end != '\0' || v == 0) return kLogPool;
-  return unsigned(std::min<unsigned long>(v, kLogPool));
-}
-
-// Voxels per reduction tile on the current device: 16384 (a 64-bit word
-// each, 128 KB of LDS), or the largest power of two its LDS per block holds.
-static int log_tile() {
-  static std::mutex mu;
-  static std::map<int, int> tiles;
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = tiles.find(dev);
-  if (it != tiles.end()) return it->second;
-  int max_lds = 0;
-  (void)hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  constexpr size_t kStatic = 512;  // the kernel's static LDS, rounded up
-  int tile = 16384;
-  while (tile > 1024 && size_t(tile) * sizeof(long long) + kStatic > size_t(max_lds)) tile >>= 1;
-  if (tile * sizeof(long long) > 65536 &&
-      hipFuncSetAttribute(reinterpret_cast<const void *>(log_reduce_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, int(tile * sizeof(long long))) != hipSuccess) {
-    (void)hipGetLastError();
-    tile = 65536 / int(sizeof(long long)) / 2;
-  }
-  tiles[dev] = tile;
-  return tile;
-}
-
-// Whether the one-box volume tracker takes a launch of integrator d on scene
-// s (an explicit samples_per_thread asks for the static launch).
-static bool takes_box(const Scene *s, const rcv_integrator_desc *d) {
-  return d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && d->max_depth != 0 && s->box_path();
 }
 
 // Work-unit split of the one-box renders: up to 64 units per pixel of at
@@ -876,57 +635,6 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
   return check_launch(fn);
 }
 
-// The scatter log of a persistent volume adjoint (buf, for the gradient of
-// `param`; -1: none, the scatter-adds stay atomics).
-struct LogLaunch {
-  LogBuf buf;
-  int param = -1;
-  int tile = 0;
-  int64_t nvox = 0;
-};
-
-// The density gradient of the first heterogeneous medium that has one goes
-// through the scatter log when its grid fits the reduction tiles and a
-// footprint (up to nx ny + nx + 1 voxels past its base) spans at most two
-// of them. Without memory for the log the scatter-adds stay atomics.
-static void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL) {
-  log.tile = log_tile();
-  for (const MediumInfo &M : s->media) {
-    if (M.homogeneous || M.sigma_param < 0 || !G.g[M.sigma_param]) continue;
-    const Param &P = s->params[M.sigma_param];
-    const int64_t n = int64_t(P.nx) * P.ny * P.nz;
-    if (n <= int64_t(log.tile) * kLogMaxTiles && n < (int64_t(1) << kRecBaseBits) &&
-        int64_t(P.nx) * P.ny + P.nx + 1 <= log.tile) {
-      log.param = M.sigma_param;
-      log.nvox = n;
-    }
-    break;
-  }
-  if (log.param >= 0 && log_buffer(stream, log.buf) != RCV_OK) {
-    (void)hipGetLastError();
-    log.param = -1;
-  }
-  if (log.param < 0) return;
-  GL.log_rec = log.buf.rec;
-  GL.log_ctl = log.buf.ctl;
-  GL.log_list = log.buf.list;
-  GL.log_fill = log.buf.fill;
-  GL.log_chunks = log_pool_chunks();
-  GL.log_shift = __builtin_ctz(unsigned(log.tile));
-  GL.log_param = log.param;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1 + kLogBins), 0, stream, log.buf.ctl);
-}
-
-static void reduce_log(const Scene *s, const GradTargets &GL, hipStream_t stream, const LogLaunch &log) {
-  if (log.param < 0) return;
-  const Param &P = s->params[log.param];
-  const int tiles = int((log.nvox + log.tile - 1) / log.tile);
-  hipLaunchKernelGGL(log_reduce_kernel, dim3(kLogSplits, tiles), dim3(kReduceBlock),
-                     size_t(log.tile) * sizeof(long long), stream, log.buf.rec, log.buf.ctl, log.buf.list,
-                     log.buf.fill, GL.log_chunks, int(P.nx), int(P.nx) * int(P.ny), log.nvox, log.tile,
-                     GL.g[log.param]);
-}
-
 int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uint32_t seed, int spp,
                    const float *grad_img, int n_params, const int32_t *param_ids, float *const *grad_ptrs,
                    hipStream_t stream) {
@@ -1008,12 +716,12 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
         // three waves per SIMD with the log, four with atomics (kWavesPerEuLoggedAdjoint)
         if constexpr (kTapeAdjoint<F>)
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
-        else if (log.param >= 0)
+        else if (log.target.g)
           go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint>);
         else
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
       });
-    reduce_log(s, GL, stream, log);
+    reduce_log(log, GL, stream);
   }
   else if (d->type == RCV_INTEGRATOR_VOLPATH)
     with_render_features(s->features(), [&](auto f) {

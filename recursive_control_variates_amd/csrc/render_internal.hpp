@@ -80,6 +80,15 @@ __host__ __device__ inline int sample_end(int c, int spp, int chunk_log2) {
   return int((int64_t(c + 1) * spp) >> chunk_log2);
 }
 
+// Camera samples per work unit of the volume path tracer's persistent
+// launches (the adjoint; the renders, within kRenderMaxUnitsPerPixel). With
+// small units the lanes of a wavefront trace samples of the same few pixels,
+// whose paths start alike and share L1 lines of the grid, and the last units
+// of a launch are short. The 64^3 adjoint at the mid / final state of the
+// optimisation: 46.1 / 67.5 ms with 16-sample units, 39.7 / 51.4 with 8,
+// 37.0 / 47.8 with 4, 36.2 / 46.4 with 2.
+constexpr int kVolUnitSamples = 2;
+
 // Render, adjoint and forward mode of the one-box volume tracker.
 constexpr int kBoxRender = 0;
 constexpr int kBoxAdjoint = 1;
@@ -113,6 +122,25 @@ struct BoxLaunch {
   float *partial;
   unsigned *queue;
 };
+BoxScene bound_box(const Scene *s);  // the tracker's scene with the bound states
+
+// Whether the one-box volume tracker takes a launch of integrator d on scene
+// s (an explicit samples_per_thread asks for the static launch).
+inline bool takes_box(const Scene *s, const rcv_integrator_desc *d) {
+  return d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && d->max_depth != 0 && s->box_path();
+}
+
+// Calls fn with the compile-time feature mask of a one-box scene.
+template <typename Fn>
+inline void with_box_features(int f, Fn &&fn) {
+  switch (f & (kFeatAlbedoGrid | kFeatSupergrid)) {
+    case 0: fn(std::integral_constant<int, 0>{}); break;
+    case kFeatAlbedoGrid: fn(std::integral_constant<int, kFeatAlbedoGrid>{}); break;
+    case kFeatSupergrid: fn(std::integral_constant<int, kFeatSupergrid>{}); break;
+    default: fn(std::integral_constant<int, kFeatAlbedoGrid | kFeatSupergrid>{}); break;
+  }
+}
+
 void launch_box(const Scene *s, int ns, int mode, const BoxLaunch &L);
 
 int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint32_t seed, int spp,

@@ -366,12 +366,18 @@ int Scene::upload(hipStream_t stream) {
   const size_t o_q = put(q_init, sizeof(q_init));
 
   RCV_TRY_HIP(hipMalloc(&dev_block, blob.size()), "rcv_scene_commit: hipMalloc");
+  // the scenes of the one-box tracker
+  one_box = shapes.size() == 1 && box_shape.size() == 1 && tri_shape.empty() && sph_shape.empty() &&
+            media.size() == 1 && !media[0].homogeneous && media[0].sample_emitters && shapes[0].interior == 0 &&
+            shapes[0].exterior == -1 && shapes[0].emitter < 0 && shapes[0].bsdf >= 0 &&
+            bsdfs[shapes[0].bsdf].type == RCV_BSDF_NULL && emitters.size() == 1 &&
+            emitters[0].type == RCV_EMITTER_CONSTANT;
   // unit sums of persistent renders: up to kRenderMaxUnitsPerPixel units of
   // (old, new) RGB per pixel of the largest sensor
   {
     int64_t max_pix = 0;
     for (auto &sen : sensors) max_pix = std::max(max_pix, int64_t(sen.film_w) * sen.film_h);
-    partial_cap = std::max(max_pix * kRenderMaxUnitsPerPixel, std::min(max_pix * 64, kRenderMinUnits)) * 6;
+    partial_cap = std::max(max_pix * kRenderMaxUnitsPerPixel, one_box ? std::min(max_pix * 64, kRenderMinUnits) : 0) * 6;
     if (partial_cap > 0)
       RCV_TRY_HIP(hipMalloc(&partial, size_t(partial_cap) * sizeof(float)), "rcv_scene_commit: hipMalloc");
   }
@@ -436,11 +442,6 @@ int Scene::upload(hipStream_t stream) {
     }
   }
   n_nodes = int(b.nodes.size());
-  one_box = shapes.size() == 1 && box_shape.size() == 1 && tri_shape.empty() && sph_shape.empty() &&
-            media.size() == 1 && !media[0].homogeneous && media[0].sample_emitters && shapes[0].interior == 0 &&
-            shapes[0].exterior == -1 && shapes[0].emitter < 0 && shapes[0].bsdf >= 0 &&
-            bsdfs[shapes[0].bsdf].type == RCV_BSDF_NULL && emitters.size() == 1 &&
-            emitters[0].type == RCV_EMITTER_CONSTANT;
   if (one_box) {
     box_scene.root = b.nodes[0];
     box_scene.box = boxes[0];

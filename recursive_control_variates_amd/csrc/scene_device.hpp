@@ -404,11 +404,18 @@ struct GridFoot {
   __device__ int idx(int c) const { return base + ((c & 1) ? dx : 0) + ((c & 2) ? dy : 0) + ((c & 4) ? dz : 0); }
 };
 
-__device__ inline void grid_footprint(const ParamBind &P, const MediumInfo &M, V3 p, GridFoot &g) {
+// Voxel coordinate of a relative position l in [0, 1] along an axis of n
+// voxels. (Fused in every kernel: a point's footprint is formed again from
+// the point where the scatter log is added up.)
+__device__ inline float voxel_coord(float l, int n) { return __builtin_fmaf(l, float(n), -0.5f); }
+
+// (P: a ParamBind or LogTarget; M: a MediumInfo or LogTarget)
+template <class Grid, class Box>
+__device__ inline void grid_footprint(const Grid &P, const Box &M, V3 p, GridFoot &g) {
   const float lx = (p.x - M.lo[0]) / (M.hi[0] - M.lo[0]);
   const float ly = (p.y - M.lo[1]) / (M.hi[1] - M.lo[1]);
   const float lz = (p.z - M.lo[2]) / (M.hi[2] - M.lo[2]);
-  const float x = lx * float(P.nx) - 0.5f, y = ly * float(P.ny) - 0.5f, z = lz * float(P.nz) - 0.5f;
+  const float x = voxel_coord(lx, P.nx), y = voxel_coord(ly, P.ny), z = voxel_coord(lz, P.nz);
   const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
   g.tx = x - fx;
   g.ty = y - fy;

@@ -15,9 +15,10 @@ namespace rcv {
 // state of the optimisation 15.9 / 21.5 -> 12.6 / 15.8 ms, 3.1 -> 3.7 ms at
 // the uniform initial state (eight: 12.3 / 14.8, 4.4 ms).
 constexpr int kRenderMaxUnitsPerPixel = 4;
-// Small images may be split further, into up to 64 units per pixel, as long
-// as the buffer stays within this many units (25 MB).
-constexpr int64_t kRenderMinUnits = int64_t(1) << 20;
+// Small images of the one-box tracker's scenes may be split further, into up
+// to 64 units per pixel, as long as the buffer stays within this many units
+// (6 MB; one per lane the device holds).
+constexpr int64_t kRenderMinUnits = int64_t(1) << 18;
 
 struct Param {
   int kind = 0;

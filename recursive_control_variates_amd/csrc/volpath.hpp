@@ -24,41 +24,56 @@
 namespace rcv {
 
 // Scatter log geometry: reduction tiles of a logged gradient, bins (one per
-// tile, then one per seam between tiles t and t + 1), records per chunk.
+// tile, then one per seam between tiles t and t + 1; the last seam does not
+// exist), records per chunk, chunks a wavefront draws from the pool at once.
 constexpr int kLogMaxTiles = 16;
 constexpr int kLogBins = 2 * kLogMaxTiles;
 constexpr unsigned kLogChunk = 256;
+constexpr unsigned kLogDraw = 8;
+constexpr int kLogFillBits = 9;  // log_meta: record count (<= kLogChunk) in the low bits, bin above
+static_assert(kLogChunk < (1u << kLogFillBits), "a chunk's record count fits its bits");
 
 struct GradTargets {
   float *g[kMaxParams];
-  // Scatter log (the persistent volume adjoint): the replay pass appends
-  // each scatter-add into g[log_param] as a record in log_rec (log_record)
-  // instead of adding it. Records
-  // are binned by the reduction tile (2^log_shift voxels) their corners
-  // fall in: bin t for tile t, bin kLogMaxTiles + t for footprints across
-  // tiles t and t + 1. A wavefront fills chunks of kLogChunk records, one
-  // per bin at a time, drawn from a pool of log_chunks: log_ctl[0] counts
-  // the chunks drawn, log_ctl[1 + b] those of bin b, listed in
-  // log_list[b * log_chunks + k]; log_fill[c] is chunk c's record count.
-  // log_reduce_kernel adds the records up. Null log_rec: scatter-adds are
-  // atomics.
-  int4 *log_rec;
+  // Scatter log (the persistent volume adjoints): the replay pass appends
+  // each scatter-add into g[log_param] as a record (point, value) in log_rec
+  // instead of adding it. Records are binned by the reduction tile
+  // (2^log_shift voxels) their corners fall in: bin t for tile t, bin
+  // kLogMaxTiles + t for footprints across tiles t and t + 1. A wavefront
+  // fills chunks of kLogChunk records, one per bin at a time, drawn kLogDraw
+  // at a time from a pool of log_chunks: *log_ctl counts the chunks drawn,
+  // log_meta[c] holds chunk c's bin (log_bin0 + bin, so that several
+  // gradients share a pool) and record count. log_reduce_kernel adds the
+  // records up. Null log_rec: scatter-adds are atomics.
+  float4 *log_rec;
   unsigned *log_ctl;
-  unsigned *log_list;
-  unsigned *log_fill;
+  unsigned *log_meta;
   unsigned log_chunks;
+  unsigned log_bin0;
   int log_shift;
   int log_param;
   __host__ __device__ void clear() {
     for (int i = 0; i < kMaxParams; ++i) g[i] = nullptr;
     log_rec = nullptr;
     log_ctl = nullptr;
-    log_list = nullptr;
-    log_fill = nullptr;
+    log_meta = nullptr;
     log_chunks = 0;
+    log_bin0 = 0;
     log_shift = 0;
     log_param = -1;
   }
+};
+
+// A gradient whose scatter-adds are logged, for the reduction: the grid, its
+// placement (footprints are formed again from the records' points), the
+// first bin of its chunks and the first of its tiles among those of all
+// gradients of the launch.
+struct LogTarget {
+  float *g;
+  int nx, ny, nz;
+  float lo[3], hi[3];
+  unsigned bin0;
+  int tile0;
 };
 
 // Event counters of a launch (scene counting mode): each call adds n per
@@ -360,64 +375,69 @@ __device__ inline bool pack_cell(const GridFoot &f, int medium, unsigned &cell) 
 
 __device__ inline int cell_medium(unsigned cell) { return int(cell >> 29); }
 
-// A scatter log record, 16 B: the packed footprint (pack_cell), the three
-// fractions as 21-bit fixed point (round((2^21 - 1) t); a fraction lies in
-// [0, 1]) in 63 bits, and the value.
-constexpr float kLogFracScale = 2097151.0f;
-
-__device__ inline int4 log_record(unsigned cell, const GridFoot &f, float val) {
-  const unsigned long long q = (unsigned long long)__float2uint_rn(f.tx * kLogFracScale) |
-                               ((unsigned long long)__float2uint_rn(f.ty * kLogFracScale) << 21) |
-                               ((unsigned long long)__float2uint_rn(f.tz * kLogFracScale) << 42);
-  return make_int4(int(cell), int(unsigned(q)), int(unsigned(q >> 32)), __float_as_int(val));
-}
-
 // Scatter log state of the lane's wavefront, in LDS word
 // kLdsWordsPerThread - 1 of its lanes (free in every scene: past the stack,
 // and past the NEE weights, which leave the last slot free): lane b holds
 // the chunk the wavefront fills for bin b (-1: none), lane kLogBins + b
-// that chunk's record count. Only the wavefront itself touches them.
+// that chunk's record count; in the place of the last bin, which no
+// footprint has, the next and the end of the chunks it has drawn. Only the
+// wavefront itself touches them.
 static_assert(2 * kLogBins == 64, "scatter log state: two words per bin in a wavefront's 64 lanes");
+constexpr int kLogNext = kLogBins - 1, kLogEnd = 2 * kLogBins - 1;
 
 __device__ inline int *wave_log_word(const LdsStack &L, int lane) {
   return L.base + (kLdsWordsPerThread - 1) * L.stride - int(threadIdx.x & 63u) + lane;
 }
 
-// Before the wavefront's first scatter: no chunk in any bin.
-__device__ inline void log_begin(const GradTargets &G, const LdsStack &L) {
-  const int lane = int(threadIdx.x & 63u);
-  if (G.log_rec) *wave_log_word(L, lane) = lane < kLogBins ? -1 : 0;
+__device__ inline unsigned log_meta_of(const GradTargets &G, int bin, unsigned fill) {
+  return ((G.log_bin0 + unsigned(bin)) << kLogFillBits) | min(fill, kLogChunk);
 }
 
-// With the whole wavefront past its last scatter: the record counts of the
-// chunks it still fills.
-__device__ inline void log_end(const GradTargets &G, const LdsStack &L) {
+// Before the wavefront's first scatter: no chunk in any bin, none drawn.
+__device__ inline void log_begin(const GradTargets &G, const LdsStack &L) {
   const int lane = int(threadIdx.x & 63u);
-  if (G.log_rec && lane < kLogBins) {
+  if (G.log_rec) *wave_log_word(L, lane) = lane < kLogNext ? -1 : 0;
+}
+
+// With the whole wavefront past its last scatter into G's gradient: the
+// chunks it still fills are closed.
+__device__ inline void log_close(const GradTargets &G, const LdsStack &L) {
+  const int lane = int(threadIdx.x & 63u);
+  if (G.log_rec && lane < kLogNext) {
     const int c = *wave_log_word(L, lane);
-    if (c >= 0) G.log_fill[c] = unsigned(*wave_log_word(L, kLogBins + lane));
+    if (c >= 0) G.log_meta[c] = log_meta_of(G, lane, unsigned(*wave_log_word(L, kLogBins + lane)));
+    *wave_log_word(L, lane) = -1;
+    *wave_log_word(L, kLogBins + lane) = 0;
   }
 }
 
-// Scatter-add of val over footprint f into the gradient of param. When
-// that gradient is logged the record goes to its bin's current chunk, at
-// the slot an LDS atomic on the bin's count gives the lane. Lanes left
-// without a slot (the chunk is full, or the bin has none yet) are rare:
-// for the bin of the first of them the chunk is closed (its count stored)
-// and the next one drawn from the pool with one global atomic, and those
-// of any other bin add with atomics this once. Added with atomics
-// otherwise, once the pool is used up, or for a footprint that does not
-// pack.
+// After log_close, at the wavefront's end: the chunks it drew and did not
+// use are empty.
+__device__ inline void log_end(const GradTargets &G, const LdsStack &L) {
+  if (!G.log_rec) return;
+  const unsigned next = unsigned(*wave_log_word(L, kLogNext));
+  const unsigned end = min(unsigned(*wave_log_word(L, kLogEnd)), G.log_chunks);
+  for (unsigned c = next + (threadIdx.x & 63u); c < end; c += 64) G.log_meta[c] = 0;
+}
+
+// Scatter-add of val over footprint f (of point p) into the gradient of
+// param. When that gradient is logged the record goes to its bin's current
+// chunk, at the slot an LDS atomic on the bin's count gives the lane. Lanes
+// left without a slot (the chunk is full, or the bin has none yet) are rare:
+// for the bin of the first of them the chunk is closed and the wavefront's
+// next one opened (drawn from the pool with one global atomic for kLogDraw
+// chunks: the pool's counter is one address for all XCDs), and those of any
+// other bin add with atomics this once. Added with atomics otherwise, and
+// once the pool is used up.
 __device__ inline void scatter_density(const GradTargets *G, const LdsStack &L, int param, float *g,
-                                       const GridFoot &f, float val) {
-  unsigned cell;
-  if (G->log_rec == nullptr || param != G->log_param || !pack_cell(f, 0, cell)) {
+                                       const GridFoot &f, V3 p, float val) {
+  if (G->log_rec == nullptr || param != G->log_param) {
     scatter_grid(g, f, val);
     return;
   }
   const int tile = f.base >> G->log_shift;
   const int bin = ((f.base + f.dx + f.dy + f.dz) >> G->log_shift) == tile ? tile : kLogMaxTiles + tile;
-  const int4 rec = log_record(cell, f, val);
+  const float4 rec = make_float4(p.x, p.y, p.z, val);
   const int chunk = *wave_log_word(L, bin);
   const unsigned r = unsigned(__hip_atomic_fetch_add(wave_log_word(L, kLogBins + bin), 1, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_WAVEFRONT));
@@ -436,12 +456,15 @@ __device__ inline void scatter_density(const GradTargets *G, const LdsStack &L, 
   if (lane == leader) {
     int *const cw = wave_log_word(L, b);
     int *const fw = wave_log_word(L, kLogBins + b);
-    if (*cw >= 0) G->log_fill[*cw] = min(unsigned(*fw), kLogChunk);
-    const unsigned id = atomicAdd(G->log_ctl, 1u);
-    if (id < G->log_chunks) {
-      c = int(id);
-      G->log_list[size_t(b) * G->log_chunks + atomicAdd(G->log_ctl + 1 + b, 1u)] = id;
+    if (*cw >= 0) G->log_meta[*cw] = log_meta_of(*G, b, unsigned(*fw));
+    unsigned next = unsigned(*wave_log_word(L, kLogNext));
+    const unsigned end = unsigned(*wave_log_word(L, kLogEnd));
+    if (next >= end && end < G->log_chunks) {  // (no draw once the pool's end is known)
+      next = atomicAdd(G->log_ctl, kLogDraw);
+      *wave_log_word(L, kLogEnd) = int(next + kLogDraw);
     }
+    if (next < G->log_chunks) c = int(next);
+    *wave_log_word(L, kLogNext) = int(next + 1);
     *cw = c;
     *fw = c >= 0 ? int(__popcll(mb)) : 0;
   }
@@ -592,7 +615,7 @@ __device__ inline bool shadow_step(const SceneView &S, Shadow<NS> &sh, SurfInt &
         if (fwd_sum) {
           *fwd_sum += -M.scale / mev.sn[NS - 1] * grid_eval1(g, mev.foot);
         } else {
-          scatter_density(G, stack, M.sigma_param, g, mev.foot, -gscale * M.scale / mev.sn[NS - 1]);
+          scatter_density(G, stack, M.sigma_param, g, mev.foot, mev.p, -gscale * M.scale / mev.sn[NS - 1]);
           cnt.add(kCntGradAtomics, 8);
         }
       }
@@ -1257,9 +1280,9 @@ struct VolPath {
         }
       } else if (gd && lr != 0.0f) {
         if (act_null) {
-          if (mev.sn[0] != 0.0f) scatter_density(G, stack, M.sigma_param, gd, mev.foot, -lr * M.scale / mev.sn[0]);
+          if (mev.sn[0] != 0.0f) scatter_density(G, stack, M.sigma_param, gd, mev.foot, mev.p, -lr * M.scale / mev.sn[0]);
         } else {
-          scatter_density(G, stack, M.sigma_param, gd, mev.foot, lr * M.scale / mev.st[0]);
+          scatter_density(G, stack, M.sigma_param, gd, mev.foot, mev.p, lr * M.scale / mev.st[0]);
         }
         cnt.add(kCntGradAtomics, 8);
       }

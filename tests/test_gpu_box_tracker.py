@@ -112,3 +112,37 @@ def test_box_tracker_empty_and_masked(cuda):
     img = integ.render(sc, 0, 3, spp)
     env = torch.tensor([1.0, 0.7, 1.4], device="cuda")
     np.testing.assert_allclose(img.cpu().numpy(), env.expand_as(img).cpu().numpy(), rtol=1e-5)
+
+
+@pytest.mark.parametrize("many_pixels", [False, True])
+def test_batched_box_jobs_equal_single_launches(cuda, monkeypatch, many_pixels):
+    # first iteration of a batch of every feature mask (old = new = initial
+    # value), one job plain: images and gradients of the single launches with
+    # the same seeds; with many pixels the renders' units are whole pixels
+    from recursive_control_variates_amd.batch import BatchOptimizer, JobSpec
+    from recursive_control_variates_amd.rendering import sample_tea_32
+    announce(f"batched one-box jobs vs single launches (many_pixels={many_pixels})")
+    w, h = (760, 240) if many_pixels else (37, 23)
+    specs, want = [], []
+    for i, k in enumerate([0, 3, 4, 6, 7]):
+        sc, p, integ, _, _, spp, _ = _scene(CASES[k], w, h)
+        init = p[SIGMA].detach().clone()
+        for _ in range(2):
+            for key in p.keys():
+                p[key] = p[key].detach().clone().requires_grad_(key == SIGMA)
+            p.update()
+        seed = 100 + i
+        img = (integ.render(sc, 0, seed, spp) if i == 1 else integ.render_twostates(sc, 0, seed, spp)[1])
+        ref = torch.full_like(img, 0.4)
+        g = integ.adjoint(sc, p, 2.0 * (img - ref) / img.numel(), 0, sample_tea_32(seed, 1)[0], spp)[SIGMA]
+        want.append((img.cpu().numpy(), g.cpu().numpy()))
+        specs.append(JobSpec(scene=sc, key=SIGMA, init=init, img_ref=ref, method="baseline" if i == 1 else "cv_ps",
+                             integrator=dict(CASES[k][5], type="twostateprbvolpath"), loss="L2", spp=spp, seed=seed))
+    batch = BatchOptimizer(specs, use_graph=False)
+    batch.step(1)
+    batch.synchronize()
+    for j, (img, g) in enumerate(want):
+        np.testing.assert_allclose(batch.image(j).cpu().numpy(), img, rtol=1e-5, atol=1e-6)
+        got = batch.jobs[j].grad.cpu().numpy()
+        assert np.allclose(got, g, rtol=1e-4, atol=1e-5 * np.abs(g).max()), (j, np.abs(got - g).max())
+    batch.close()
