@@ -294,14 +294,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
           for (int s = sample_end(chunk - 1, J.spp_g, J.cl2_g); s < s_end; ++s) {
             Pcg32 rng = lane_rng(seed, uint32_t(pixel * J.spp_g + s));
             const Ray ray = camera_ray(sen, px, py, rng);
-            const Pcg32 rng0 = rng;
-            V3 L[1];
-            path_sample<1, false>(S, J.integ, rng, ray, L, stack, cnt, nullptr, nullptr);
-            if (!any_nonzero(L[0])) continue;
-            AdjState adj{dL, L[0]};
-            rng = rng0;
-            V3 L2[1];
-            path_sample<1, true>(S, J.integ, rng, ray, L2, stack, cnt, &adj, &J.gt);
+            path_adjoint_sample(S, J.integ, rng, ray, dL, J.gt, stack, cnt);
           }
         }
       }

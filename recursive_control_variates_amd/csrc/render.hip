@@ -92,33 +92,26 @@ __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(kWave
   }
 }
 
-// The adjoint of camera sample s of a pixel for the per-sample integrators
-// (surface path tracer, volpathsimple): the primal pass, then the adjoint pass
-// with the same random numbers -- a replay that scatters d(log weight)/d(theta)
-// times the radiance still to come (path tracer, skipped when L = 0), or
-// volpathsimple's adjoint with its gradient-only stream as well (DRT
-// contributes even where L = 0).
+// The adjoint of camera sample s of a pixel for the per-sample integrators:
+// the surface path tracer's (path_adjoint_sample), or volpathsimple's primal
+// pass, then its adjoint with the same random numbers and its gradient-only
+// stream (DRT contributes even where L = 0).
 template <int INTEG, int F>
 __device__ inline void adjoint_one_sample(const SceneView &S, const IntegArgs &I, const SensorInfo &sen,
                                           uint32_t seed, int px, int py, int64_t pixel, int spp, int s, V3 dL,
                                           const GradTargets &G, const LdsStack &stack, LocalCounters &cnt) {
   Pcg32 rng = lane_rng(seed, uint32_t(pixel * spp + s));
   const Ray ray = camera_ray(sen, px, py, rng);
-  const Pcg32 rng0 = rng;
-  V3 L[1];
   if constexpr (INTEG == RCV_INTEGRATOR_VOLPATH_SIMPLE) {
+    const Pcg32 rng0 = rng;
+    V3 L[1];
     L[0] = simple_sample<false, F>(S, I, 0, rng, ray, simple_camera_start(), stack, cnt, nullptr, nullptr, nullptr);
     AdjState adj{dL, L[0]};
     rng = rng0;
     Pcg32 alt = lane_rng(simple_alt_seed(seed), uint32_t(pixel * spp + s));
     (void)simple_sample<true, F>(S, I, 0, rng, ray, simple_camera_start(), stack, cnt, &adj, &alt, &G);
   } else {
-    path_sample<1, false>(S, I, rng, ray, L, stack, cnt, nullptr, nullptr);
-    if (!any_nonzero(L[0])) return;
-    AdjState adj{dL, L[0]};
-    rng = rng0;
-    V3 L2[1];
-    path_sample<1, true>(S, I, rng, ray, L2, stack, cnt, &adj, &G);
+    path_adjoint_sample(S, I, rng, ray, dL, G, stack, cnt);
   }
 }
 
