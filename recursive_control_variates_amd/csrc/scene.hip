@@ -10,6 +10,7 @@
 // order-independent atomic max, so no host synchronisation is needed.
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -185,6 +186,71 @@ __global__ __launch_bounds__(256) void max_reduce_kernel(const float *__restrict
 
 }  // namespace
 
+// The planar primitives of a scene of few triangles: pairs of consecutive
+// triangles of a shape that form a parallelogram, and the other triangles. In
+// double, from the triangles' float corners. Empty when there are more than
+// kMaxFlat of them, or one is degenerate.
+static std::vector<FlatPrim> flat_prims(const std::vector<float> &tri_v, const std::vector<int32_t> &tri_shape,
+                                        const std::vector<int32_t> &slot_of) {
+  std::vector<FlatPrim> out;
+  const int n = int(tri_shape.size());
+  using P = std::array<double, 3>;
+  auto corner = [&](int t, int c) { return P{tri_v[9 * t + 3 * c], tri_v[9 * t + 3 * c + 1], tri_v[9 * t + 3 * c + 2]}; };
+  auto sub = [](P a, P b) { return P{a[0] - b[0], a[1] - b[1], a[2] - b[2]}; };
+  auto dot3 = [](P a, P b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
+  auto cross3 = [](P a, P b) {
+    return P{a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
+  };
+  for (int t = 0; t < n;) {
+    P p = corner(t, 0), a = sub(corner(t, 1), p), b = sub(corner(t, 2), p);
+    int other = -1;
+    if (t + 1 < n && tri_shape[t + 1] == tri_shape[t]) {
+      // corner i of t and corner j of t + 1 opposite their common edge
+      for (int i = 0; i < 3 && other < 0; ++i)
+        for (int j = 0; j < 3 && other < 0; ++j) {
+          const P s1 = corner(t, (i + 1) % 3), s2 = corner(t, (i + 2) % 3);
+          const P r1 = corner(t + 1, (j + 1) % 3), r2 = corner(t + 1, (j + 2) % 3);
+          if (!((s1 == r1 && s2 == r2) || (s1 == r2 && s2 == r1))) continue;
+          const P pi = corner(t, i), pj = corner(t + 1, j);
+          const P d = {pi[0] + pj[0] - s1[0] - s2[0], pi[1] + pj[1] - s1[1] - s2[1], pi[2] + pj[2] - s1[2] - s2[2]};
+          const P e = sub(s1, s2);
+          if (dot3(d, d) > 1e-12 * dot3(e, e)) continue;
+          p = pi;
+          a = sub(s1, pi);
+          b = sub(s2, pi);
+          other = t + 1;
+        }
+    }
+    const P m = cross3(a, b);
+    const double len = std::sqrt(dot3(m, m));
+    if (!(len > 1e-10) || int(out.size()) == kMaxFlat) return {};
+    const P nn = {m[0] / len, m[1] / len, m[2] / len};
+    // dual basis: A . a = 1, A . b = 0, A . n = 0
+    P A = cross3(b, nn), B = cross3(nn, a);
+    const double ka = 1.0 / dot3(A, a), kb = 1.0 / dot3(B, b);
+    FlatPrim f{};
+    for (int k = 0; k < 3; ++k) {
+      A[k] *= ka;
+      B[k] *= kb;
+      f.n[k] = float(nn[k]);
+      f.A[k] = float(A[k]);
+      f.B[k] = float(B[k]);
+    }
+    f.nd = float(dot3(nn, p));
+    f.a0 = float(-dot3(A, p));
+    f.b0 = float(-dot3(B, p));
+    const P C = {A[0] + B[0], A[1] + B[1], A[2] + B[2]};
+    f.la = float(1.0 / std::sqrt(dot3(A, A)));
+    f.lb = float(1.0 / std::sqrt(dot3(B, B)));
+    f.lc = float(1.0 / std::sqrt(dot3(C, C)));
+    f.slot0 = slot_of[t];
+    f.slot1 = other >= 0 ? slot_of[other] : -1;
+    out.push_back(f);
+    t += other >= 0 ? 2 : 1;
+  }
+  return out;
+}
+
 int Scene::upload(hipStream_t stream) {
   // ---- primitives
   const int n_tris = int(tri_v.size() / 9);
@@ -290,6 +356,10 @@ int Scene::upload(hipStream_t stream) {
     sphere_shape_v[s] = sph_shape[s];
   }
 
+  // ---- planar primitives of a small scene
+  const std::vector<FlatPrim> flat = n_box == 0 && n_sph <= kMaxFlatSpheres ? flat_prims(tri_v, tri_shape, slot_of)
+                                                                            : std::vector<FlatPrim>();
+
   // ---- area emitters: triangle CDF per emitter
   std::vector<float> em_cdf;
   std::vector<int32_t> em_tris;
@@ -357,6 +427,7 @@ int Scene::upload(hipStream_t stream) {
   const size_t o_cdf = put(em_cdf.data(), em_cdf.size() * 4);
   const size_t o_emt = put(em_tris.data(), em_tris.size() * 4);
   const size_t o_med = put(media.data(), media.size() * sizeof(MediumInfo));
+  const size_t o_flat = put(flat.data(), flat.size() * sizeof(FlatPrim));
   const size_t o_sens = put(sensors.data(), sensors.size() * sizeof(SensorInfo));
   std::vector<uint32_t> maj_init(2 * kMaxParams, float_key(-kInf));
   const size_t o_maj = put(maj_init.data(), maj_init.size() * 4);
@@ -407,6 +478,11 @@ int Scene::upload(hipStream_t stream) {
   counters = reinterpret_cast<unsigned long long *>(base + o_cnt);
   work_queue = reinterpret_cast<unsigned *>(base + o_q);
   v.counters = nullptr;
+  v.flat = reinterpret_cast<const FlatPrim *>(base + o_flat);
+  v.n_flat = int(flat.size());
+  v.flat_extent = 0.0f;
+  for (int k = 0; k < 3; ++k) v.flat_extent = std::max(v.flat_extent, std::max(std::fabs(all.lo[k]), std::fabs(all.hi[k])));
+  for (int i = 0; i < kMaxFlatSpheres; ++i) v.flat_sph_slot[i] = i < n_sph ? slot_of[n_tris + i] : -1;
   v.n_tris = n_tris;
   v.n_sph = n_sph;
   v.n_emitters = int(emitters.size());

@@ -214,10 +214,121 @@ __device__ inline LdsStack lds_of(const SceneView &S, int *lds) {
   return LdsStack{lds + tid, stride, lds + S.lds_stack * stride + tid, S.lds_slots};
 }
 
+// trace() over the planar primitives and spheres of a small scene (SceneView::
+// n_flat), all of them for every ray: no divergence, no stack, and the
+// primitives' data in scalar registers. What bounds the surface tracer is
+// instruction issue, and a BVH over a dozen primitives spends more of it on
+// boxes, with half the lanes masked off, than this takes for the
+// primitives (Cornell box, 512^2, 32 samples, depth 6: two-state render
+// 5.8 -> 2.8 ms, adjoint 6.9 -> 4.4 ms).
+//
+// The result is the BVH's bit for bit: plane and edge tests in plain
+// arithmetic only decide which primitive is hit, and only when they decide it
+// beyond their own rounding error (`eps`, a bound of the position error) and
+// beyond that of the exact triangle test; then that test gives the hit. -1
+// for a ray nearer to an edge, a diagonal, a plane or a tie than that: the
+// caller takes the BVH.
+template <bool ANY_HIT>
+__device__ inline int flat_trace(const SceneView &S, const Ray &r, Hit &h) {
+  h.slot = -1;
+  h.t = kInf;
+  // errors of positions grow with the largest coordinate in play, of the
+  // crossing with 1 / |n . d|; 8e-6 is ~100 roundings of it
+  const float scale = fmaxf(S.flat_extent, fmaxf(fabsf(r.o.x), fmaxf(fabsf(r.o.y), fabsf(r.o.z))));
+  const float e0 = 8e-6f * scale;
+  float best = kInf, best_eps = 0.0f, best_w = 0.0f;  // nearest sure hit, its error, its distance to the diagonal
+  float other = kInf;                                 // lower bound of every other hit, sure or not
+  int slot0 = -1, slot1 = -1;
+  bool occluded = false;
+  const auto *prims = reinterpret_cast<const __attribute__((address_space(4))) FlatPrim *>(
+      reinterpret_cast<uintptr_t>(S.flat));
+  for (int i = 0; i < S.n_flat; ++i) {
+    const FlatPrim f = *(const FlatPrim *)(prims + i);
+    const float nd = f.n[0] * r.d.x + f.n[1] * r.d.y + f.n[2] * r.d.z;
+    const float no = f.nd - (f.n[0] * r.o.x + f.n[1] * r.o.y + f.n[2] * r.o.z);
+    const float inv = __builtin_amdgcn_rcpf(nd);
+    const float t = no * inv;
+    const float eps = e0 + e0 * fabsf(inv);
+    const float u = f.a0 + (f.A[0] * r.o.x + f.A[1] * r.o.y + f.A[2] * r.o.z) +
+                    t * (f.A[0] * r.d.x + f.A[1] * r.d.y + f.A[2] * r.d.z);
+    const float v = f.b0 + (f.B[0] * r.o.x + f.B[1] * r.o.y + f.B[2] * r.o.z) +
+                    t * (f.B[0] * r.d.x + f.B[1] * r.d.y + f.B[2] * r.d.z);
+    // distance to the nearest edge, positive inside
+    const float w = (1.0f - u - v) * f.lc;
+    float m = f.slot1 >= 0 ? fminf((0.5f - fabsf(u - 0.5f)) * f.la, (0.5f - fabsf(v - 0.5f)) * f.lb)
+                           : fminf(fminf(u * f.la, v * f.lb), w);
+    // surely missed: outside, behind the origin or past the end
+    const bool missed = m < -eps || t + eps < 0.0f || t - eps > r.maxt;
+    const bool hit = m > eps && t - eps > 0.0f && t + eps < r.maxt;
+    if (ANY_HIT && hit) occluded = true;
+    if (!missed) {
+      const float lo = t - eps;
+      if (!hit) {
+        other = lo < other ? lo : (lo == lo ? other : -kInf);  // (NaN: undecided)
+      } else if (t < best) {
+        other = fminf(other, best - best_eps);
+        best = t;
+        best_eps = eps;
+        best_w = w;
+        slot0 = f.slot0;
+        slot1 = f.slot1;
+      } else {
+        other = fminf(other, lo);
+      }
+    }
+  }
+  for (int i = 0; i < S.n_sph; ++i) {
+    float t;
+    const float4 sp = S.spheres[i];
+    const bool hit = hit_sphere(sp, r, r.maxt, t);
+    // a ray that grazes the sphere may miss its bounds in the BVH
+    const V3 fo = r.o - v3(sp.x, sp.y, sp.z);
+    const V3 l = fo - r.d * dot(fo, r.d);
+    const bool grazing = fabsf(sp.w * sp.w - dot(l, l)) < 1e-3f * sp.w * sp.w;
+    if (grazing) other = -kInf;
+    if (!hit) continue;
+    if (ANY_HIT && !grazing) occluded = true;
+    if (t < best) {
+      other = fminf(other, best - best_eps);
+      best = t;
+      best_eps = 0.0f;
+      slot0 = S.flat_sph_slot[i];
+      slot1 = -2;
+    } else {
+      other = fminf(other, t);
+    }
+  }
+  if (ANY_HIT) {
+    if (occluded) return 1;
+    return other == kInf ? 0 : -1;
+  }
+  if (best == kInf) return other == kInf ? 0 : -1;
+  if (!(best + best_eps < other)) return -1;
+  if (slot1 == -2) {
+    h.t = best;
+    h.slot = slot0;
+    h.b1 = h.b2 = 0.0f;
+    return 1;
+  }
+  if (slot1 >= 0 && !(fabsf(best_w) > best_eps)) return -1;
+  const int slot = slot1 >= 0 && best_w < 0.0f ? slot1 : slot0;
+  float t, b1, b2;
+  if (!hit_triangle(S.tris, slot, r, r.maxt, t, b1, b2)) return -1;
+  h.t = t;
+  h.slot = slot;
+  h.b1 = b1;
+  h.b2 = b2;
+  return 1;
+}
+
 // Closest hit (any_hit = false) or occlusion test (any_hit = true) against
 // [0, r.maxt). Stack depth never exceeds the BVH depth (SceneView::lds_stack).
 template <bool ANY_HIT>
 __device__ inline bool trace(const SceneView &S, const Ray &r, Hit &h, const LdsStack &stack) {
+  if (S.n_flat > 0) {
+    const int found = flat_trace<ANY_HIT>(S, r, h);
+    if (found >= 0) return found != 0;
+  }
   const V3 inv_d = v3(1.0f / r.d.x, 1.0f / r.d.y, 1.0f / r.d.z);
   float tbest = r.maxt;
   h.slot = -1;

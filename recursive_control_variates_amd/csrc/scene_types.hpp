@@ -59,6 +59,22 @@ struct BoxPrim {
   int32_t pad;
 };
 
+// A planar primitive of a small scene (scene_device.hpp, flat_trace): a
+// parallelogram of two triangles (slot0 holds the corner u + v < 1, slot1 the
+// other) or one triangle (slot1 = -1). With the plane n . p = nd, a point p of
+// it has u = A . p + a0, v = B . p + b0; la, lb (and lc, for u + v = 1) turn a
+// difference in u, v or u + v into a distance.
+struct FlatPrim {
+  float n[3], nd;
+  float A[3], a0;
+  float B[3], b0;
+  float la, lb, lc;
+  int32_t slot0, slot1;
+  int32_t pad;
+};
+constexpr int kMaxFlat = 16;
+constexpr int kMaxFlatSpheres = 4;
+
 struct ShapeInfo {
   int32_t bsdf;      // -1: none
   int32_t emitter;   // -1: none
@@ -143,6 +159,10 @@ struct SceneView {
   const float *majorants;    // [param][state] max of the grid data
   const float *supergrids;   // per-medium supergrid majorants (two states)
   unsigned long long *counters;  // kNumCounters or null
+  const FlatPrim *flat;      // small scenes: their planar primitives (n_flat; 0: use the BVH)
+  int32_t flat_sph_slot[kMaxFlatSpheres];
+  float flat_extent;         // largest coordinate of the scene
+  int32_t n_flat;
   int32_t n_tris;
   int32_t n_sph;
   int32_t n_emitters;
