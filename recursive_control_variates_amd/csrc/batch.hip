@@ -75,13 +75,13 @@ __global__ void batch_rotate_kernel(BatchJobDev *jobs, int n_jobs, unsigned *que
 }
 
 // ----------------------------------------------------------- 1b. supergrid
-// One thread per (job, state, cell) over the jobs whose optimised grid has a
+// One wavefront per (job, state, cell) over the jobs whose optimised grid has a
 // majorant supergrid; ends[] are the cumulative 2 * cells counts.
 __global__ void batch_supergrid_kernel(const BatchJobDev *__restrict__ jobs, const int32_t *__restrict__ ids,
                                        const int64_t *__restrict__ ends, int n, int64_t total) {
-  const int64_t u = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t u = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (u >= total) return;
-  const int k = find_job(ends, n, u);
+  const int k = __builtin_amdgcn_readfirstlane(find_job(ends, n, u));
   const BatchJobDev &J = jobs[ids[k]];
   if (!J.active) return;
   const int cells = J.sg_res[0] * J.sg_res[1] * J.sg_res[2];
@@ -89,8 +89,8 @@ __global__ void batch_supergrid_kernel(const BatchJobDev *__restrict__ jobs, con
   const int state = local >= cells ? RCV_STATE_NEW : RCV_STATE_OLD;
   const int c = local - (state == RCV_STATE_NEW ? cells : 0);
   const ParamBind &P = J.view.params[J.param];
-  J.sg_out[state * cells + c] =
-      supergrid_cell_max(P.data[state], P.nx, P.ny, P.nz, J.sg_res[0], J.sg_res[1], J.sg_res[2], c);
+  const float m = supergrid_cell_max(P.data[state], P.nx, P.ny, P.nz, J.sg_res[0], J.sg_res[1], J.sg_res[2], c);
+  if ((threadIdx.x & 63u) == 0) J.sg_out[state * cells + c] = m;
 }
 
 // ---------------------------------------------------------------- 2. render
@@ -747,7 +747,7 @@ static int enqueue_step(rcv_batch *b, hipStream_t st) {
                      b->d_queues);
   if (!b->sg_ids.empty()) {
     const int64_t total = b->sg_ends.back();
-    hipLaunchKernelGGL(batch_supergrid_kernel, dim3(ceil_div(total, 128)), dim3(128), 0, st, b->d_jobs,
+    hipLaunchKernelGGL(batch_supergrid_kernel, dim3(ceil_div(total, 4)), dim3(256), 0, st, b->d_jobs,
                        b->d_sg_ids, b->d_sg_ends, int(b->sg_ids.size()), total);
   }
   // render classes: (path, 1), (path, 2), (vol, 1), (vol, 2); queues 0..3 reused per class in sequence

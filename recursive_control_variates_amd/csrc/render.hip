@@ -689,6 +689,12 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     const int ucl2 = unit_chunk_log2(spp, cl2, taped ? kAdjUnitSamples : kVolUnitSamples);
     const unsigned units = unsigned(n_pix << ucl2);
     GradTargets GL = G;
+    // only constants of the homogeneous medium to differentiate
+    const int hom = s->view.hom_medium;
+    GL.hom_once = hom >= 0;
+    for (int i = 0; i < n_params; ++i)
+      if (hom < 0 || (param_ids[i] != s->media[hom].sigma_param && param_ids[i] != s->media[hom].albedo_param))
+        GL.hom_once = false;
     LogLaunch log;
     if (!taped) open_log(s, G, stream, log, GL);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
@@ -706,10 +712,11 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
           hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
                              ucl2, grad_img, GL, s->work_queue, units);
         };
-        // three waves per SIMD with the log, four with atomics (kWavesPerEuLoggedAdjoint)
+        // three waves per SIMD with the log or without scatter-adds, four
+        // with atomics (kWavesPerEuLoggedAdjoint)
         if constexpr (kTapeAdjoint<F>)
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
-        else if (log.target.g)
+        else if (log.target.g || GL.hom_once)
           go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint>);
         else
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
@@ -779,11 +786,13 @@ int launch_forward(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
 }
 
 namespace {
-__global__ void supergrid_kernel(const float *__restrict__ grid, int nx, int ny, int nz, int sx, int sy, int sz,
-                                 float *__restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// A wavefront per cell.
+__global__ __launch_bounds__(256) void supergrid_kernel(const float *__restrict__ grid, int nx, int ny, int nz, int sx,
+                                                        int sy, int sz, float *__restrict__ out) {
+  const int c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (c >= sx * sy * sz) return;
-  out[c] = supergrid_cell_max(grid, nx, ny, nz, sx, sy, sz, c);
+  const float m = supergrid_cell_max(grid, nx, ny, nz, sx, sy, sz, c);
+  if ((threadIdx.x & 63u) == 0) out[c] = m;
 }
 }  // namespace
 
@@ -792,7 +801,7 @@ int Scene::build_supergrid(int medium, int state, hipStream_t stream) {
   const Param &p = params[m.sigma_param];
   const int cells = m.sg_res[0] * m.sg_res[1] * m.sg_res[2];
   float *out = supergrids + m.supergrid_offset + state * cells;
-  hipLaunchKernelGGL(supergrid_kernel, dim3(ceil_div(cells, 128)), dim3(128), 0, stream, p.data[state], p.nx, p.ny,
+  hipLaunchKernelGGL(supergrid_kernel, dim3(ceil_div(cells, 4)), dim3(256), 0, stream, p.data[state], p.nx, p.ny,
                      p.nz, m.sg_res[0], m.sg_res[1], m.sg_res[2], out);
   return check_launch("majorant supergrid");
 }

@@ -164,21 +164,31 @@ inline uint32_t float_key(float f) {
 
 __global__ void fill_u32_kernel(uint32_t *p, uint32_t v) { *p = v; }
 
-__global__ __launch_bounds__(256) void max_reduce_kernel(const float *__restrict__ x, int64_t n,
-                                                         uint32_t *__restrict__ out) {
-  __shared__ float red[256];
+// A block ends with an atomic on the one result, ~15 ns each one after the
+// other: 13.8 us for a 64^3 grid in 1024 blocks, 4.4 us in at most 256.
+constexpr int kMaxReduceBlocks = 256;
+
+__global__ __launch_bounds__(1024) void max_reduce_kernel(const float *__restrict__ x, int64_t n,
+                                                          uint32_t *__restrict__ out) {
+  __shared__ float red[16];
   float m = -kInf;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x)
-    m = fmaxf(m, x[i]);
-  red[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (int(threadIdx.x) < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
-    __syncthreads();
+  const int64_t first = int64_t(blockIdx.x) * blockDim.x + threadIdx.x, stride = int64_t(gridDim.x) * blockDim.x;
+  int64_t i = first;
+  if ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    for (; i < n / 4; i += stride) {
+      const float4 v = x4[i];
+      m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+    }
+    i = n / 4 * 4 + first;
   }
+  for (; i < n; i += stride) m = fmaxf(m, x[i]);
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, red[0]);
+    for (int w = 1; w < int(blockDim.x >> 6); ++w) m = fmaxf(m, red[w]);
+    const uint32_t u = __builtin_bit_cast(uint32_t, m);
     const uint32_t key = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
     atomicMax(out, key);
   }
@@ -547,8 +557,8 @@ int Scene::reduce_param(int param, int state, hipStream_t stream) {
   const int64_t n = int64_t(p.nx) * p.ny * p.nz * p.ch;
   uint32_t *slot = majorant_keys + 2 * param + state;
   hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(1), 0, stream, slot, float_key(-kInf));
-  const unsigned grid = unsigned(std::min<int64_t>(1024, (n + 255) / 256));
-  hipLaunchKernelGGL(max_reduce_kernel, dim3(grid), dim3(256), 0, stream, p.data[state], n, slot);
+  const unsigned grid = unsigned(std::min<int64_t>(kMaxReduceBlocks, (n + 4095) / 4096));
+  hipLaunchKernelGGL(max_reduce_kernel, dim3(grid), dim3(1024), 0, stream, p.data[state], n, slot);
   int rc = check_launch("rcv_scene_bind_param: majorant reduction");
   if (rc != RCV_OK) return rc;
   for (int mi = 0; mi < int(media.size()); ++mi)

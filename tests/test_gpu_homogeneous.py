@@ -196,3 +196,30 @@ def test_tutorial_optimisation_loop(cuda):
     assert np.isfinite(losses).all()
     assert final > 1.0          # moved from 0.2 towards the target
     assert np.mean(losses[-10:]) < np.mean(losses[:10])
+
+
+@pytest.mark.parametrize("max_depth", [3, 16])
+def test_one_pass_adjoint_is_the_transpose_of_forward_mode(cuda, max_depth):
+    # the persistent adjoint of the homogeneous constants sums its terms in
+    # the primal pass; forward mode replays every path of the same samples
+    announce(f"one-pass homogeneous adjoint vs forward mode (max_depth {max_depth})")
+    from recursive_control_variates_amd import scenes
+    rng = np.random.default_rng(max_depth)
+    sc = rcv.load_dict(scenes.homogeneous_cornell_scene_dict(sigma_t=0.7, film_res=32, spp=8, albedo=(0.6, 0.8, 0.9)))
+    p = rcv.traverse(sc)
+    key_a = scenes.HOMOGENEOUS_KEY.replace("sigma_t", "albedo")
+    for k in (scenes.HOMOGENEOUS_KEY, key_a):
+        p[k] = p[k].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    integ = rcv.load_dict({"type": "prbvolpath", "max_depth": max_depth, "rr_depth": 6})
+    g = torch.from_numpy(rng.uniform(0.5, 1.5, (32, 32, 3)).astype(np.float32)).cuda()
+    grads = integ.adjoint(sc, p, g, 0, 5, 8)
+    for k in (scenes.HOMOGENEOUS_KEY, key_a):
+        t = torch.from_numpy(rng.uniform(0.5, 1.0, tuple(p[k].shape)).astype(np.float32)).cuda()
+        fwd = integ.render_forward(sc, p, 0, 5, 8, tangents={k: t}).double()
+        lhs = float((g.double() * fwd).sum())
+        rhs = float((grads[k].double() * t.double()).sum())
+        # terms of both signs: float32 rounding of their absolute sum
+        size = float((g.double() * fwd.abs()).sum())
+        assert size > 0 and abs(lhs - rhs) <= 1e-5 * size, (k, lhs, rhs, size)
