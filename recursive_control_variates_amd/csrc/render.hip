@@ -272,7 +272,12 @@ adjoint_persistent_kernel(SceneView S, IntegArgs I, int sensor, uint32_t seed, i
 // (a pixel's chunk of camera samples) from a device counter and run
 // adjoint_one_sample for each, so long pixels do not hold their wavefronts at
 // the end of the launch. The result per sample is that of adjoint_kernel;
-// only the order of the gradient scatter-adds differs.
+// only the order of the gradient scatter-adds differs. volpathsimple's density
+// scatter-adds go through the log where it is set: each is a 16-byte record
+// in place of 8 atomics, and a sample has ~50 of them (64^3, 128^2, 16
+// samples, majorant supergrid: 6.1 ms and 0.5 ms of reduction against 7.5 ms
+// with atomics). What is
+// left is issue in the nested tracking loops, whose lanes diverge.
 template <int INTEG, int F>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<INTEG>))) void
 adjoint_sample_persistent_kernel(
@@ -283,6 +288,8 @@ adjoint_sample_persistent_kernel(
   const SensorInfo &sen = S.sensors[sensor];
   const int film_w = sen.film_w;
   LocalCounters cnt{S.counters};
+  constexpr bool kLogs = INTEG == RCV_INTEGRATOR_VOLPATH_SIMPLE;
+  if constexpr (kLogs) log_begin(G, stack);
   int s = 0, s_end = 0, px = 0, py = 0;
   int64_t pixel = 0;
   V3 dL = v3(0.f);
@@ -311,6 +318,11 @@ adjoint_sample_persistent_kernel(
     }
     adjoint_one_sample<INTEG, F>(S, I, sen, seed, px, py, pixel, spp, s, dL, G, stack, cnt);
     ++s;
+  }
+  // the whole wavefront is past its loop
+  if constexpr (kLogs) {
+    log_close(G, stack);
+    log_end(G, stack);
   }
 }
 
@@ -661,20 +673,24 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
   // the per-sample integrators' persistent adjoint, as the volume path
   // tracer's below
-  auto launch_sample_persistent = [&](auto kern) {
+  auto launch_sample_persistent = [&](auto kern, const GradTargets &targets) {
     const int ucl2 = unit_chunk_log2(spp, cl2, kAdjUnitSamples);
     const unsigned units = unsigned(n_pix << ucl2);
     const unsigned pgrid =
         std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)), ceil_div(int64_t(units), block));
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
     hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp, ucl2,
-                       grad_img, G, s->work_queue, units);
+                       grad_img, targets, s->work_queue, units);
   };
-  if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE && !d->samples_per_thread)
+  if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE && !d->samples_per_thread) {
+    GradTargets GL = G;
+    LogLaunch log;
+    open_log(s, G, stream, log, GL, n_pix * spp, kSimpleLogSamples);
     with_volume_features(s->features(), [&](auto f) {
-      launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>);
+      launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>, GL);
     });
-  else if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE)
+    reduce_log(log, GL, stream);
+  } else if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE)
     with_volume_features(s->features(), [&](auto f) {
       hipLaunchKernelGGL((adjoint_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>), dim3(grid),
                          dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp, spt, cl2, grad_img,
@@ -729,7 +745,7 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
                          stack_bytes(block), stream, s->view, I, sensor, seed, spp, spt, cl2, grad_img, G);
     });
   else if (!d->samples_per_thread)
-    launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_PATH, 0>);
+    launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_PATH, 0>, G);
   else
     hipLaunchKernelGGL((adjoint_kernel<RCV_INTEGRATOR_PATH, 0>), dim3(grid), dim3(block), stack_bytes(block), stream,
                        s->view, I, sensor, seed, spp, spt, cl2, grad_img, G);

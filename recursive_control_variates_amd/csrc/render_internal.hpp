@@ -64,6 +64,15 @@ template <int NS, int INTEG>
 constexpr int kWavesPerEuRender = INTEG == RCV_INTEGRATOR_VOLPATH && NS == 2 ? 3 : kWavesPerEu<INTEG>;
 constexpr int kWavesPerEuLoggedAdjoint = 3;
 
+// Camera samples per reduction tile from which volpathsimple's adjoint logs
+// its density scatter-adds. A launch too small to fill the device waits for
+// its longest path, which hides the atomics, and the reduction costs ~5 us a
+// tile: adjoint with atomics / logged, 64^3 (16 tiles) with 64 Ki samples
+// 1.18 / 1.23 ms, 96 Ki 2.08 / 2.08, 128 Ki 1.65 / 1.55, 256 Ki 2.67 / 2.16;
+// 48^3 (7 tiles) with 32 Ki 1.13 / 1.13, 64 Ki 1.18 / 1.15, 128 Ki 1.70 /
+// 1.39; 32^3 (2 tiles) with 16 Ki 1.11 / 1.08, 64 Ki 1.30 / 1.13.
+constexpr int64_t kSimpleLogSamples = 8192;
+
 // Splits the spp camera samples of a pixel over 2^chunk_log2 threads (at
 // most spt samples each): a user-given samples_per_thread must divide spp
 // into a power of two <= 64 chunks; otherwise chunks double, up to the

@@ -187,6 +187,8 @@ int allocate(LogBuf &out) {
 
 // The pool of single launches: one per (device, stream), kept for the
 // process (launches on one stream run in order; other streams get their own).
+// None is allocated while the stream is being captured, which an allocation
+// would break off: a launch captured before any other has no log.
 int stream_pool(hipStream_t stream, LogBuf &out) {
   static std::mutex mu;
   static std::map<std::pair<int, hipStream_t>, LogBuf> bufs;
@@ -196,6 +198,12 @@ int stream_pool(hipStream_t stream, LogBuf &out) {
   const auto key = std::make_pair(dev, stream);
   auto it = bufs.find(key);
   if (it == bufs.end()) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+      (void)hipGetLastError();
+      return 1;
+    }
+    if (capture != hipStreamCaptureStatusNone) return 1;
     LogBuf nb;
     if (int rc = allocate(nb)) return rc;
     it = bufs.emplace(key, nb).first;
@@ -275,11 +283,12 @@ void log_into(const LogBuf &buf, int param, unsigned bin0, GradTargets &G) {
   G.log_param = param;
 }
 
-void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL) {
+void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL,
+              int64_t samples, int64_t min_samples) {
   for (const MediumInfo &M : s->media) {
     if (M.homogeneous || M.sigma_param < 0 || !G.g[M.sigma_param]) continue;
     log.tiles = log_target(s, M, G.g[M.sigma_param], log.target);
-    if (log.tiles > 0 && stream_pool(stream, log.buf) == RCV_OK) {
+    if (log.tiles > 0 && samples >= min_samples * log.tiles && stream_pool(stream, log.buf) == RCV_OK) {
       log_into(log.buf, M.sigma_param, 0, GL);
       hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, stream, log.buf.ctl);
     } else {

@@ -38,8 +38,10 @@ void log_into(const LogBuf &buf, int param, unsigned bin0, GradTargets &G);
 
 // Sets up the log of a launch on `stream` for the density gradient of the
 // first heterogeneous medium that has one, with the stream's pool. Without
-// memory for it the scatter-adds stay atomics.
-void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL);
+// memory for it, or with fewer than `min_samples` (per reduction tile) of the
+// launch's `samples`, the scatter-adds stay atomics.
+void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL,
+              int64_t samples = 0, int64_t min_samples = 0);
 
 // Adds the records of a launch to its gradient.
 void reduce_log(const LogLaunch &log, const GradTargets &GL, hipStream_t stream);

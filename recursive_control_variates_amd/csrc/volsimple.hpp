@@ -43,6 +43,15 @@ constexpr int kSimpleNoDrt = RCV_SIMPLE_NO_DRT;
 constexpr int kSimpleNoDrtSubsampling = RCV_SIMPLE_NO_DRT_SUBSAMPLING;
 constexpr int kSimpleNoDrtMis = RCV_SIMPLE_NO_DRT_MIS;
 
+// The tentative collisions of a shadow ray that its replay would scatter at,
+// recorded so that they can be once the NEE's contribution is known: point
+// and d log(weight)/d(density). The footprint is formed again from the point,
+// which is also what the scatter log keeps.
+struct SimpleNeeRecord {
+  int n;  // kNeeRecords + 1: overflowed, and the shadow ray is tracked again
+  float4 e[kNeeRecords];
+};
+
 // Tentative collisions with the majorant until a real one (accepted with
 // probability sigma_t / majorant) or the end of the segment
 // (sample_real_interaction, plugins/volpathsimple.py:315-367). `ev.t` is
@@ -71,12 +80,11 @@ __device__ inline void simple_real_collision(const SceneView &S, int medium, Ray
 // (estimate_transmittance, plugins/volpathsimple.py:450-491). GRAD: scatter
 // -adj * scale / sigma_n per tentative collision (the replay of :476-482).
 // rec (adjoint, first pass): the collisions that replay would scatter at
-// (point, sigma_n; sigma_n = 0 where it would not), so the caller can scatter
-// them once adj is known.
+// (SimpleNeeRecord), so the caller can scatter them once adj is known.
 template <int F, bool GRAD>
 __device__ inline float simple_ratio_tracking(const SceneView &S, int medium, Ray ray, float tmax, Pcg32 &rng,
                                               LocalCounters &cnt, float adj, const GradTargets *G,
-                                              NeeRecord *rec = nullptr) {
+                                              const LdsStack &stack, SimpleNeeRecord *rec = nullptr) {
   float T = 1.0f;
   ray.maxt = tmax;
   while (true) {
@@ -89,16 +97,13 @@ __device__ inline float simple_ratio_tracking(const SceneView &S, int medium, Ra
       const MediumInfo &M = S.media[medium];
       float *g = G->g[M.sigma_param];
       if (g && adj != 0.0f) {
-        scatter_grid(g, ev.foot, -adj * M.scale / ev.sn[0]);
+        scatter_density(G, stack, M.sigma_param, g, ev.foot, ev.p, -adj * M.scale / ev.sn[0]);
         cnt.add(kCntGradAtomics, 8);
       }
     }
-    if (rec) {
-      unsigned cell;
-      if (rec->n < kNeeRecords && pack_cell(ev.foot, medium, cell)) {
-        rec->e[rec->n] = make_float4(ev.foot.tx, ev.foot.ty, ev.foot.tz,
-                                     tr > 0.0f ? -S.media[medium].scale / ev.sn[0] : 0.0f);
-        rec->cell[rec->n] = cell;
+    if (rec && tr > 0.0f) {
+      if (rec->n < kNeeRecords) {
+        rec->e[rec->n] = make_float4(ev.p.x, ev.p.y, ev.p.z, -S.media[medium].scale / ev.sn[0]);
         rec->n++;
       } else {
         rec->n = kNeeRecords + 1;
@@ -118,7 +123,7 @@ __device__ inline float simple_ratio_tracking(const SceneView &S, int medium, Ra
 template <int F, bool GRAD>
 __device__ inline V3 simple_sample_emitter(const SceneView &S, int medium, V3 p, Pcg32 &rng, DirSample &ds,
                                            const LdsStack &stack, LocalCounters &cnt, float adj,
-                                           const GradTargets *G, NeeRecord *rec = nullptr) {
+                                           const GradTargets *G, SimpleNeeRecord *rec = nullptr) {
   const float u1 = rng.next_1d();
   const float u2 = rng.next_1d();
   V3 ev = sample_emitter_direction(S, p, u1, u2, ds);
@@ -132,7 +137,7 @@ __device__ inline V3 simple_sample_emitter(const SceneView &S, int medium, V3 p,
   cnt.add(kCntTraversals, 1);
   const SurfInt si = make_si(S, r, h);
   if (!si.valid) return v3(0.f);
-  return ev * simple_ratio_tracking<F, GRAD>(S, medium, r, si.t, rng, cnt, adj, G, rec);
+  return ev * simple_ratio_tracking<F, GRAD>(S, medium, r, si.t, rng, cnt, adj, G, stack, rec);
 }
 
 // Where a path starts: from the camera (cross the medium boundary first,
@@ -282,7 +287,8 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
           const V3 dl = adj->dL * li;
           float *gd = G->g[M.sigma_param];
           if (gd) {
-            scatter_grid(gd, mev.foot, mis * dot(dl, albedo) * M.scale / mev.st[0]);
+            scatter_density(G, stack, M.sigma_param, gd, mev.foot, mev.p,
+                            mis * dot(dl, albedo) * M.scale / mev.st[0]);
             cnt.add(kCntGradAtomics, 8);
           }
           if ((F & kFeatAlbedoGrid) && M.albedo_param >= 0 && G->g[M.albedo_param]) {
@@ -303,8 +309,9 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
           const float tj = alt->next_1d() * interval;
           if (gd && lr != 0.0f && interval < kInf) {
             GridFoot f;
-            grid_footprint(P, M, ray_at(ray, tj), f);
-            scatter_grid(gd, f, -lr * M.scale * interval * 0.25f);
+            const V3 pj = ray_at(ray, tj);
+            grid_footprint(P, M, pj, f);
+            scatter_density(G, stack, M.sigma_param, gd, f, pj, -lr * M.scale * interval * 0.25f);
             cnt.add(kCntGradAtomics, 8);
           }
         }
@@ -322,7 +329,7 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
     if (use_nee && did_scatter && active) {
       const Pcg32 nee_rng = rng;
       DirSample ds;
-      NeeRecord rec;
+      SimpleNeeRecord rec;
       rec.n = 0;
       const V3 em = simple_sample_emitter<F, false>(S, medium, mev.p, rng, ds, stack, cnt, 0.0f, G,
                                                     ADJ ? &rec : nullptr);
@@ -336,14 +343,14 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
           DirSample ds2;
           if (rec.n <= kNeeRecords) {
             // the replay's scatter-adds, from the recorded collisions
-            RecMedium rm;
-            rm.select(S, G, medium);
-            for (int j = 0; rm.g && j < rec.n; ++j) {
+            float *const gd = G->g[M.sigma_param];
+            for (int j = 0; gd && j < rec.n; ++j) {
               const float4 e = rec.e[j];
-              if (e.w != 0.0f) {
-                scatter_grid(rm.g, rm.foot(e, rec.cell[j]), cs * e.w);
-                cnt.add(kCntGradAtomics, 8);
-              }
+              const V3 pj = v3(e.x, e.y, e.z);
+              GridFoot f;
+              grid_footprint(S.params[M.sigma_param], M, pj, f);
+              scatter_density(G, stack, M.sigma_param, gd, f, pj, cs * e.w);
+              cnt.add(kCntGradAtomics, 8);
             }
           } else {
             (void)simple_sample_emitter<F, true>(S, medium, mev.p, r2, ds2, stack, cnt, cs, G);
@@ -442,7 +449,7 @@ __device__ void simple_drt(const SceneView &S, const IntegArgs &I, int medium, R
   seg.o = ray_at(ray, mint);
   seg.d = ray.d;
   seg.maxt = kInf;
-  const float T = simple_ratio_tracking<F, false>(S, medium, seg, s, alt, cnt, 0.0f, G);
+  const float T = simple_ratio_tracking<F, false>(S, medium, seg, s, alt, cnt, 0.0f, G, stack);
   const float weight = pdf > 0.0f ? T / pdf : 0.0f;
   const V3 p = ray_at(ray, mint + s);
   const ParamBind &P = S.params[M.sigma_param];
@@ -463,7 +470,7 @@ __device__ void simple_drt(const SceneView &S, const IntegArgs &I, int medium, R
   const V3 a = adjoint * li * (mis * weight);
   float *gd = G->g[M.sigma_param];
   if (gd && weight != 0.0f) {
-    scatter_grid(gd, foot, dot(a, alb) * M.scale);
+    scatter_density(G, stack, M.sigma_param, gd, foot, p, dot(a, alb) * M.scale);
     cnt.add(kCntGradAtomics, 8);
   }
   if ((F & kFeatAlbedoGrid) && M.albedo_param >= 0 && G->g[M.albedo_param] && weight != 0.0f) {

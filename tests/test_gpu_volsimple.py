@@ -135,3 +135,43 @@ def test_adjoint_integrator_of_a_cv_optimisation(cuda):
     assert np.isfinite(res["param_mse"]).all()
     assert res["param_mse"][-1] < res["param_mse"][0]
     assert bool(torch.isfinite(res["final"][KEY]).all())
+
+
+# A grid inside one reduction tile of the scatter log, several tiles whose
+# seams cut through slices, rows of one voxel past a power of two; with the
+# majorant supergrid; each DRT form; and a pool that runs out.
+@pytest.mark.parametrize("shape,factor,props,chunks", [
+    ((9, 7, 5), 0, {}, None),
+    ((40, 48, 48), 8, {}, None),
+    ((33, 17, 65), 0, {"use_drt_subsampling": False}, None),
+    ((40, 48, 48), 0, {"use_drt": False}, None),
+    ((24, 24, 24), 4, {"use_nee": False}, None),
+    ((40, 48, 48), 0, {}, "40"),
+])
+def test_logged_adjoint_equals_atomics(cuda, monkeypatch, shape, factor, props, chunks):
+    # The persistent launch logs the density scatter-adds, the static one
+    # (samples_per_thread) adds them with float atomics; the samples are the
+    # same (98304 of them: enough for the log to be taken on every grid here).
+    # A voxel gets at most a few thousand terms; the rounding errors of their
+    # float sums in two orders add up like a random walk to ~sqrt(4000) 2^-24 =
+    # 4e-6 of the largest gradient, times 5 for the cancellation of signs.
+    announce(f"volpathsimple adjoint, scatter log vs atomics {shape} factor {factor} {props} pool {chunks}")
+    if chunks:
+        monkeypatch.setenv("RCV_SCATTER_LOG_CHUNKS", chunks)
+    rng = np.random.default_rng(41)
+    grid = (0.2 + rng.uniform(0, 0.8, shape + (1,))).astype(np.float32)
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=0.8, scale=5.0, w=48, h=32, spp=64, majorant_factor=factor))
+    gimg = torch.from_numpy(rng.uniform(0.5, 1.5, (32, 48, 3)).astype(np.float32)).cuda()
+    integ = rcv.load_dict(dict({"type": "volpathsimple", "max_depth": 8, "rr_depth": 4}, **props))
+    p = rcv.traverse(sc)
+    p[KEY] = p[KEY].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    grads = []
+    for spt in (0, 4):
+        integ.samples_per_thread = spt
+        grads.append(integ.adjoint(sc, p, gimg, 0, 43, 64)[KEY].double().cpu().numpy())
+    a, b = grads
+    scale = np.abs(b).max()
+    assert scale > 0 and (b != 0).mean() > 0.5, (b != 0).mean()
+    assert np.allclose(a, b, rtol=1e-4, atol=2e-5 * scale), np.abs(a - b).max() / scale
