@@ -686,9 +686,17 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     GradTargets GL = G;
     LogLaunch log;
     open_log(s, G, stream, log, GL, n_pix * spp, kSimpleLogSamples);
-    with_volume_features(s->features(), [&](auto f) {
-      launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>, GL);
-    });
+    if (takes_simple_box(s, d)) {
+      const int ucl2 = unit_chunk_log2(spp, cl2, kVolUnitSamples);
+      hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+      launch_simple_box(s, BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), grad_img, &GL,
+                                     nullptr, s->work_queue});
+    } else {
+      with_volume_features(s->features(), [&](auto f) {
+        launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>,
+                                 GL);
+      });
+    }
     reduce_log(log, GL, stream);
   } else if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE)
     with_volume_features(s->features(), [&](auto f) {

@@ -67,10 +67,12 @@ constexpr int kWavesPerEuLoggedAdjoint = 3;
 // Camera samples per reduction tile from which volpathsimple's adjoint logs
 // its density scatter-adds. A launch too small to fill the device waits for
 // its longest path, which hides the atomics, and the reduction costs ~5 us a
-// tile: adjoint with atomics / logged, 64^3 (16 tiles) with 64 Ki samples
-// 1.18 / 1.23 ms, 96 Ki 2.08 / 2.08, 128 Ki 1.65 / 1.55, 256 Ki 2.67 / 2.16;
-// 48^3 (7 tiles) with 32 Ki 1.13 / 1.13, 64 Ki 1.18 / 1.15, 128 Ki 1.70 /
-// 1.39; 32^3 (2 tiles) with 16 Ki 1.11 / 1.08, 64 Ki 1.30 / 1.13.
+// tile. On the tracker (simplebox.hpp), a call with atomics / logged: 64^3 (16
+// tiles) with 16 Ki samples 1.05 / 1.11 ms, 64 Ki 1.03 / 1.05, 128 Ki 1.45 /
+// 1.21; 48^3 (7 tiles) with 16 Ki 1.07 / 1.06, 32 Ki 1.02 / 1.02; 32^3 (2
+// tiles) with 1 Ki 0.97 / 0.92, 16 Ki 1.05 / 1.05. The general kernel: 64^3
+// with 64 Ki 1.18 / 1.23, 96 Ki 2.08 / 2.08, 128 Ki 1.65 / 1.55, 256 Ki 2.67 /
+// 2.16; 48^3 with 64 Ki 1.18 / 1.15.
 constexpr int64_t kSimpleLogSamples = 8192;
 
 // Splits the spp camera samples of a pixel over 2^chunk_log2 threads (at
@@ -139,6 +141,17 @@ inline bool takes_box(const Scene *s, const rcv_integrator_desc *d) {
   return d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && d->max_depth != 0 && s->box_path();
 }
 
+// Whether the tracker takes volpathsimple's adjoint (simplebox.hpp): the
+// default estimator.
+inline bool takes_simple_box(const Scene *s, const rcv_integrator_desc *d) {
+  return d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE && !d->samples_per_thread && s->box_path() &&
+         !(d->flags & (RCV_SIMPLE_NO_NEE | RCV_SIMPLE_NO_DRT | RCV_SIMPLE_NO_DRT_SUBSAMPLING));
+}
+
+// Waves per SIMD of volpathsimple's adjoint on the tracker: four, which its
+// LDS allows (64^3 step: 6.61 ms, with three 6.61 ms).
+constexpr int kSimpleBoxWaves = 4;
+
 // Calls fn with the compile-time feature mask of a one-box scene.
 template <typename Fn>
 inline void with_box_features(int f, Fn &&fn) {
@@ -151,6 +164,7 @@ inline void with_box_features(int f, Fn &&fn) {
 }
 
 void launch_box(const Scene *s, int ns, int mode, const BoxLaunch &L);
+void launch_simple_box(const Scene *s, const BoxLaunch &L);
 
 int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint32_t seed, int spp,
                   float *img_old, float *img_new, int ns, hipStream_t stream, const char *fn);

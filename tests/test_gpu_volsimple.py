@@ -175,3 +175,49 @@ def test_logged_adjoint_equals_atomics(cuda, monkeypatch, shape, factor, props, 
     scale = np.abs(b).max()
     assert scale > 0 and (b != 0).mean() > 0.5, (b != 0).mean()
     assert np.allclose(a, b, rtol=1e-4, atol=2e-5 * scale), np.abs(a - b).max() / scale
+
+
+# One-voxel axes' neighbours, an uneven grid, the majorant supergrid, an
+# albedo grid; one bounce; Russian roulette from the first; more shadow rays
+# than weights are kept of (a dense medium of albedo 1); without DRT's MIS.
+@pytest.mark.parametrize("shape,factor,albedo,scale,depth,rr,props", [
+    ((3, 4, 2), 0, 0.8, 5.0, 8, 8, {}),
+    ((21, 13, 30), 4, "grid", 5.0, 12, 4, {}),
+    ((16, 16, 16), 0, "grid", 5.0, -1, 0, {}),
+    ((16, 16, 16), 0, 0.8, 5.0, 1, 8, {}),
+    ((16, 16, 16), 8, 1.0, 30.0, 40, 40, {}),
+    ((16, 16, 16), 0, 0.6, 8.0, 16, 2, {"use_drt_mis": False}),
+])
+def test_one_box_adjoint_equals_general(cuda, shape, factor, albedo, scale, depth, rr, props):
+    # The persistent launch runs the one-box state machine, the static one
+    # (samples_per_thread) the general integrator; the samples, their paths
+    # and scatter-adds are the same, so only the order of the float sums
+    # differs: a voxel of these small grids gets up to ~10^5 terms, whose
+    # rounding errors add up like a random walk to sqrt(10^5) 2^-24 = 2e-5 of
+    # the largest partial sum; 1e-4 of the largest gradient allows for partial
+    # sums five times the result.
+    announce(f"volpathsimple adjoint, one-box vs general {shape} factor {factor} albedo {albedo} depth {depth} {props}")
+    rng = np.random.default_rng(47)
+    grid = (0.2 + rng.uniform(0, 0.8, shape + (1,))).astype(np.float32)
+    keys = [KEY]
+    if albedo == "grid":
+        data = rng.uniform(0.3, 0.9, shape + (3,)).astype(np.float32)
+        albedo = {"type": "gridvolume", "data": data, "to_world": T.scale(1.0)}
+        keys.append(AKEY)
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=albedo, scale=scale, w=24, h=17, spp=8, majorant_factor=factor))
+    gimg = torch.from_numpy(rng.uniform(0.5, 1.5, (17, 24, 3)).astype(np.float32)).cuda()
+    integ = rcv.load_dict(dict({"type": "volpathsimple", "max_depth": depth, "rr_depth": rr}, **props))
+    p = rcv.traverse(sc)
+    for k in keys:
+        p[k] = p[k].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    grads = []
+    for spt in (0, 4):
+        integ.samples_per_thread = spt
+        g = integ.adjoint(sc, p, gimg, 0, 53, 8)
+        grads.append([g[k].double().cpu().numpy() for k in keys])
+    for a, b in zip(*grads):
+        scale_g = np.abs(b).max()
+        assert scale_g > 0
+        assert np.allclose(a, b, rtol=1e-4, atol=1e-4 * scale_g), np.abs(a - b).max() / scale_g
