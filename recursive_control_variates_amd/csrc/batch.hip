@@ -598,13 +598,13 @@ extern "C" int rcv_batch_commit(rcv_batch *b, void *stream) {
     BatchJobDev &J = b->host_jobs[j];
     if (!b->is_box[j] || J.box.med.sigma_param != J.param) continue;
     LogTarget t;
-    const int tiles = log_target(b->scenes[j], J.box.med, J.grad, t);
+    const int tiles = log_target(b->scenes[j], J.box.med, J.grad, 0, t);
     if (tiles == 0) continue;
     if (!b->log.rec && !take_log_pool(b->log)) break;  // without memory: atomics
     t.bin0 = unsigned(kLogBins * b->log_targets.size());
     t.tile0 = b->log_tiles;
-    log_into(b->log, J.param, t.bin0, J.gt);
-    log_into(b->log, -1, 0, b->pool);
+    log_into(b->log, J.param, t.bin0, t.shift, J.gt);
+    log_into(b->log, -1, 0, t.shift, b->pool);
     b->log_tiles += tiles;
     b->log_targets.push_back(t);
   }

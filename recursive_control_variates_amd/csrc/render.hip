@@ -720,7 +720,7 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
       if (hom < 0 || (param_ids[i] != s->media[hom].sigma_param && param_ids[i] != s->media[hom].albedo_param))
         GL.hom_once = false;
     LogLaunch log;
-    if (!taped) open_log(s, G, stream, log, GL);
+    if (!taped) open_log(s, G, stream, log, GL, n_pix * spp);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
     if (box)
       launch_box(s, 1, kBoxAdjoint,

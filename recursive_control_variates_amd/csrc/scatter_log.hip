@@ -1,6 +1,7 @@
 // Scatter log of the volume adjoints: pools and reduction (GradTargets,
 // scatter_density).
 
+#include "boxpath.hpp"
 #include "scatter_log.hpp"
 
 #include <algorithm>
@@ -21,27 +22,61 @@ namespace {
 // reads the bins of its share of the chunks, 4 bytes each beside their 4 KB
 // of records.) The block looks at kReduceBlock chunks at a time, lists those
 // it takes in LDS and reads them kStepChunks per step: thread i slot i %
-// kLogChunk of kReduceUnroll of them, all loads in flight together (unused
-// slots are read, every index stays inside the pool, and skipped). The
+// kLogChunk of kReduceUnroll of them, all loads in flight together. The
 // records of one chunk come from one wavefront of the adjoint, whose lanes
 // trace neighbouring pixels; the 8-lane groups of a wavefront take their
 // chunks in rotated order so that one instruction adds records of several
 // chunks.
+//
+// A grid of more than kLogMaxTiles tiles has bins of several tiles, and each
+// of them reads its bin's records: 8 times at 128^3, whose step with an albedo
+// grid (192^2 per view, 8 samples) takes 8.8 ms (adjoint 2.8, reduction 2.2,
+// magnitudes 0.09), with atomics 11.7 (adjoint 7.2). Those bins' magnitudes
+// come from one pass over all records (log_bound_kernel) instead of one per
+// tile: 2.95 -> 2.16 ms of reduction.
+//
+// Chunks that are mostly empty (SPARSE: a short launch leaves every
+// wavefront a few records in each of up to 31 chunks) are read 64 slots of
+// kReduceUnroll chunks per wavefront instead, as long as one of them has more.
+// With bins of several tiles a block counts its records first and takes this
+// walk when fewer than half the slots are used: the 128^3 adjoint call of
+// 512 Ki thin samples 2.63 -> 1.90 ms; full chunks are read better as above
+// (that step by rows 9.1 ms).
 constexpr int kReduceBlock = 1024;
 constexpr int kReduceUnroll = 8;
 constexpr unsigned kChunkGroups = unsigned(kReduceBlock) / kLogChunk;
 constexpr unsigned kStepChunks = kChunkGroups * kReduceUnroll;
-constexpr int kLogSplits = 64;  // blocks per tile
-static_assert(kReduceBlock % int(kLogChunk) == 0, "a reduction block covers whole chunks");
+constexpr unsigned kSparseChunks = unsigned(kReduceBlock) / 64u * unsigned(kReduceUnroll);
+constexpr int kLogSplits = 64;  // blocks per tile, at most
+constexpr int kLogMinSplits = 16;
+static_assert(kReduceBlock % int(kLogChunk) == 0 && kLogChunk % 64 == 0,
+              "a reduction block covers whole chunks, a wavefront whole rows of one");
+
+// The bins whose records can reach the tile [lo, hi) of T: the one it lies in,
+// and the seams at either end of that which footprints on the tile can cross.
+struct TileBins {
+  int bin;
+  bool before, after;
+  __device__ TileBins(const LogTarget &T, int lo, int hi) : bin(lo >> T.shift) {
+    const int span = T.nx * T.ny + T.nx + 1;
+    before = bin > 0 && lo - (bin << T.shift) < span;
+    after = hi + span > ((bin + 1) << T.shift);
+  }
+  __device__ bool holds(int b) const {
+    return b == bin || (after && b == kLogMaxTiles + bin) || (before && b == kLogMaxTiles + bin - 1);
+  }
+};
 
 // Calls fn(record) for each record of the block's share that reaches `tile`.
 // picked: kReduceBlock words of LDS, n_picked one.
-template <class Fn>
+template <bool SPARSE, class Fn>
 __device__ inline void log_block_records(const float4 *__restrict__ rec, const unsigned *__restrict__ meta,
-                                         unsigned drawn, unsigned bin0, int tile, unsigned *picked,
-                                         unsigned *n_picked, Fn &&fn) {
+                                         unsigned drawn, const LogTarget &T, const TileBins &bins,
+                                         unsigned *picked, unsigned *n_picked, Fn &&fn) {
   const unsigned slot = threadIdx.x % kLogChunk;
   const unsigned sub = threadIdx.x / kLogChunk;
+  const unsigned lane = threadIdx.x & 63u;
+  const unsigned wave_sub = (threadIdx.x >> 6) * unsigned(kReduceUnroll);
   const unsigned grp = (threadIdx.x >> 3) % kReduceUnroll;
   constexpr unsigned kFillMask = (1u << kLogFillBits) - 1u;
   for (unsigned c0 = blockIdx.x; c0 < drawn; c0 += gridDim.x * unsigned(kReduceBlock)) {
@@ -49,43 +84,111 @@ __device__ inline void log_block_records(const float4 *__restrict__ rec, const u
     __syncthreads();
     const unsigned c = c0 + threadIdx.x * gridDim.x;
     const unsigned m = c < drawn ? meta[c] : 0u;
-    const int b = int(m >> kLogFillBits) - int(bin0);
-    const bool mine = (m & kFillMask) != 0 && (b == tile || b == kLogMaxTiles + tile ||
-                                               (tile > 0 && b == kLogMaxTiles + tile - 1));
+    const bool mine = (m & kFillMask) != 0 && bins.holds(int(m >> kLogFillBits) - int(T.bin0));
     if (mine) picked[atomicAdd(n_picked, 1u)] = c;
     __syncthreads();
     const unsigned nb = *n_picked;
-    for (unsigned p0 = 0; p0 < nb; p0 += kStepChunks) {
-      unsigned id[kReduceUnroll], n[kReduceUnroll];
-      float4 e[kReduceUnroll];
+    if constexpr (SPARSE) {
+      for (unsigned p0 = 0; p0 < nb; p0 += kSparseChunks) {
+        unsigned id[kReduceUnroll], n[kReduceUnroll], most = 0;
 #pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u) {
-        const unsigned j = p0 + sub + kChunkGroups * ((grp + unsigned(u)) % kReduceUnroll);
-        id[u] = j < nb ? picked[j] : picked[0];
-        n[u] = j < nb ? meta[id[u]] & kFillMask : 0u;
+        for (int u = 0; u < kReduceUnroll; ++u) {
+          const unsigned j = p0 + wave_sub + (grp + unsigned(u)) % kReduceUnroll;
+          id[u] = j < nb ? picked[j] : picked[0];
+          n[u] = j < nb ? meta[id[u]] & kFillMask : 0u;
+          most = max(most, n[u]);
+        }
+        for (unsigned row = 0; row < most; row += 64u) {
+          float4 e[kReduceUnroll];
+#pragma unroll
+          for (int u = 0; u < kReduceUnroll; ++u)
+            if (row + lane < n[u]) e[u] = rec[size_t(id[u]) * kLogChunk + row + lane];
+#pragma unroll
+          for (int u = 0; u < kReduceUnroll; ++u)
+            if (row + lane < n[u]) fn(e[u]);
+        }
       }
+    } else {
+      for (unsigned p0 = 0; p0 < nb; p0 += kStepChunks) {
+        unsigned id[kReduceUnroll], n[kReduceUnroll];
+        float4 e[kReduceUnroll];
 #pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u) e[u] = rec[size_t(id[u]) * kLogChunk + slot];
+        for (int u = 0; u < kReduceUnroll; ++u) {
+          const unsigned j = p0 + sub + kChunkGroups * ((grp + unsigned(u)) % kReduceUnroll);
+          id[u] = j < nb ? picked[j] : picked[0];
+          n[u] = j < nb ? meta[id[u]] & kFillMask : 0u;
+        }
 #pragma unroll
-      for (int u = 0; u < kReduceUnroll; ++u)
-        if (slot < n[u]) fn(e[u]);
+        for (int u = 0; u < kReduceUnroll; ++u)
+          if (slot < n[u]) e[u] = rec[size_t(id[u]) * kLogChunk + slot];
+#pragma unroll
+        for (int u = 0; u < kReduceUnroll; ++u)
+          if (slot < n[u]) fn(e[u]);
+      }
     }
     __syncthreads();
   }
 }
 
+// grid_footprint of the records' points, the extents' reciprocals formed once
+// (UniformDiv rounds as the division does, so the footprints are the same).
+struct RecordGrid {
+  UniformDiv ex, ey, ez;
+  __device__ explicit RecordGrid(const LogTarget &T)
+      : ex(T.hi[0] - T.lo[0]), ey(T.hi[1] - T.lo[1]), ez(T.hi[2] - T.lo[2]) {}
+};
+
 // Calls add(voxel - lo, value x weight) for the corners of a record that
 // fall in [lo, hi): the products of scatter_grid over the footprint of the
-// record's point.
+// record's point. A footprint without one is passed over before its weights.
 template <class Add>
-__device__ inline void record_corners(const float4 &e, const LogTarget &T, int lo, int hi, Add &&add) {
+__device__ inline void record_corners(const float4 &e, const LogTarget &T, const RecordGrid &D, int lo, int hi,
+                                      Add &&add) {
   GridFoot f;
-  grid_footprint(T, T, v3(e.x, e.y, e.z), f);
+  grid_footprint_at(T, D.ex(e.x - T.lo[0]), D.ey(e.y - T.lo[1]), D.ez(e.z - T.lo[2]), f);
+  if (f.base >= hi || f.base + f.dx + f.dy + f.dz < lo) return;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const int idx = f.idx(q);
     if (idx >= lo && idx < hi) add(idx - lo, e.w * f.w(q));
   }
+}
+
+// Largest magnitude of the records of each bin (the bits of a non-negative
+// float compare as an integer; NaN counts as inf), for a log whose bins hold
+// several tiles: one pass over the records instead of one per tile.
+constexpr int kBoundBlock = int(kLogChunk);
+constexpr int kBoundUnroll = 4;
+constexpr int kBoundBlocks = 1024;
+__global__ __launch_bounds__(kBoundBlock) void log_bound_kernel(const float4 *__restrict__ rec,
+                                                                const unsigned *__restrict__ ctl,
+                                                                const unsigned *__restrict__ meta, unsigned nchunks,
+                                                                unsigned *bound) {
+  __shared__ unsigned top[kLogBins];
+  if (threadIdx.x < unsigned(kLogBins)) top[threadIdx.x] = 0u;
+  __syncthreads();
+  const unsigned drawn = min(*ctl, nchunks);
+  constexpr unsigned kFillMask = (1u << kLogFillBits) - 1u;
+  for (unsigned c0 = blockIdx.x; c0 < drawn; c0 += gridDim.x * kBoundUnroll) {
+    unsigned m[kBoundUnroll];
+    float w[kBoundUnroll];
+#pragma unroll
+    for (int u = 0; u < kBoundUnroll; ++u) {
+      const unsigned c = c0 + unsigned(u) * gridDim.x;
+      m[u] = c < drawn ? meta[c] : 0u;
+      w[u] = threadIdx.x < (m[u] & kFillMask) ? rec[size_t(c) * kLogChunk + threadIdx.x].w : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < kBoundUnroll; ++u) {
+      const float a = fabsf(w[u]);
+      float t = a == a ? a : INFINITY;
+      for (int off = 32; off > 0; off >>= 1) t = fmaxf(t, __shfl_xor(t, off, 64));
+      if ((threadIdx.x & 63u) == 0 && t > 0.0f)
+        atomicMax(&top[(m[u] >> kLogFillBits) % unsigned(kLogBins)], __float_as_uint(t));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < unsigned(kLogBins) && top[threadIdx.x] != 0u) atomicMax(bound + threadIdx.x, top[threadIdx.x]);
 }
 
 // Adds the scatter log of a launch to its gradients, tile by tile (block y:
@@ -95,15 +198,19 @@ __device__ inline void record_corners(const float4 &e, const LogTarget &T, int l
 // largest magnitude M; terms are scaled by 2^s with M N 2^s <= 2^62, so no
 // partial sum overflows and each term is kept to ~2^-44 of M (float atomics
 // keep 2^-24 of the running sum). A share holding a non-finite value is
-// summed with float atomics as it stands.
+// summed with float atomics as it stands. WIDE: a log whose bins hold several
+// tiles; M is then its bins' (`bound`), N the share's count from its chunks.
+template <bool WIDE>
 __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *__restrict__ rec,
                                                                   const unsigned *__restrict__ ctl,
                                                                   const unsigned *__restrict__ meta, unsigned nchunks,
                                                                   LogTarget one, const LogTarget *__restrict__ many,
-                                                                  int n, int tile_voxels) {
+                                                                  int n, int tile_voxels,
+                                                                  const unsigned *__restrict__ bound) {
   extern __shared__ long long acc[];  // tile words (floats in the first half for a non-finite share)
   __shared__ float wave_max[kReduceBlock / 64];
   __shared__ unsigned wave_count[kReduceBlock / 64];
+  __shared__ unsigned wave_chunks[kReduceBlock / 64];
   __shared__ unsigned picked[kReduceBlock];
   __shared__ unsigned n_picked;
   LogTarget T = one;
@@ -116,27 +223,47 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
   const int lo = tile * tile_voxels;
   const int hi = min(lo + tile_voxels, T.nx * T.ny * T.nz);
   const unsigned drawn = min(*ctl, nchunks);
+  const TileBins bins(T, lo, hi);
+  const RecordGrid div(T);
   float m = 0.0f;
-  unsigned total = 0;
-  log_block_records(rec, meta, drawn, T.bin0, tile, picked, &n_picked, [&](const float4 &e) {
-    const float a = fabsf(e.w);
-    m = (a <= m) ? m : (a == a ? a : INFINITY);  // NaN and inf both give inf
-    ++total;
-  });
+  unsigned total = 0, chunks = 0;
+  if constexpr (WIDE) {
+    // the bins' magnitudes are known; the record count from the chunks'
+    for (unsigned c = blockIdx.x + threadIdx.x * gridDim.x; c < drawn; c += gridDim.x * unsigned(kReduceBlock)) {
+      const unsigned w = meta[c];
+      const unsigned fill = w & ((1u << kLogFillBits) - 1u);
+      if (fill != 0 && bins.holds(int(w >> kLogFillBits) - int(T.bin0))) {
+        total += fill;
+        ++chunks;
+      }
+    }
+    m = __uint_as_float(bound[bins.bin]);
+    if (bins.after) m = fmaxf(m, __uint_as_float(bound[kLogMaxTiles + bins.bin]));
+    if (bins.before) m = fmaxf(m, __uint_as_float(bound[kLogMaxTiles + bins.bin - 1]));
+  } else {
+    log_block_records<false>(rec, meta, drawn, T, bins, picked, &n_picked, [&](const float4 &e) {
+      const float a = fabsf(e.w);
+      m = (a <= m) ? m : (a == a ? a : INFINITY);  // NaN and inf both give inf
+      ++total;
+    });
+  }
   for (int off = 32; off > 0; off >>= 1) {
     m = fmaxf(m, __shfl_xor(m, off, 64));
     total += __shfl_xor(total, off, 64);
+    chunks += __shfl_xor(chunks, off, 64);
   }
   if ((threadIdx.x & 63u) == 0) {
     wave_max[threadIdx.x >> 6] = m;
     wave_count[threadIdx.x >> 6] = total;
+    wave_chunks[threadIdx.x >> 6] = chunks;
   }
   __syncthreads();
   m = 0.0f;
-  total = 0;
+  total = chunks = 0;
   for (int w = 0; w < kReduceBlock / 64; ++w) {
     m = fmaxf(m, wave_max[w]);
     total += wave_count[w];
+    chunks += wave_chunks[w];
   }
   if (total == 0 || m == 0.0f) return;
   if (isfinite(m)) {
@@ -146,11 +273,16 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
     const int sc = 62 - em - en;
     for (int v = threadIdx.x; v < tile_voxels; v += blockDim.x) acc[v] = 0;
     __syncthreads();
-    log_block_records(rec, meta, drawn, T.bin0, tile, picked, &n_picked, [&](const float4 &e) {
-      record_corners(e, T, lo, hi, [&](int a, float t) {
-        atomicAdd(reinterpret_cast<unsigned long long *>(&acc[a]), (unsigned long long)__float2ll_rn(ldexpf(t, sc)));
+    // (scaled before the weights: the same products times 2^sc)
+    auto add = [&](const float4 &e) {
+      record_corners(make_float4(e.x, e.y, e.z, ldexpf(e.w, sc)), T, div, lo, hi, [&](int a, float t) {
+        atomicAdd(reinterpret_cast<unsigned long long *>(&acc[a]), (unsigned long long)__float2ll_rn(t));
       });
-    });
+    };
+    if (WIDE && total < chunks * (kLogChunk / 2))
+      log_block_records<WIDE>(rec, meta, drawn, T, bins, picked, &n_picked, add);
+    else
+      log_block_records<false>(rec, meta, drawn, T, bins, picked, &n_picked, add);
     __syncthreads();
     for (int v = threadIdx.x; v < hi - lo; v += blockDim.x)
       if (acc[v] != 0) atomicAdd(&T.g[lo + v], ldexpf(__ll2float_rn(acc[v]), -sc));
@@ -158,8 +290,8 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
     float *facc = reinterpret_cast<float *>(acc);
     for (int v = threadIdx.x; v < tile_voxels; v += blockDim.x) facc[v] = 0.0f;
     __syncthreads();
-    log_block_records(rec, meta, drawn, T.bin0, tile, picked, &n_picked, [&](const float4 &e) {
-      record_corners(e, T, lo, hi, [&](int a, float t) { atomicAdd(&facc[a], t); });
+    log_block_records<false>(rec, meta, drawn, T, bins, picked, &n_picked, [&](const float4 &e) {
+      record_corners(e, T, div, lo, hi, [&](int a, float t) { atomicAdd(&facc[a], t); });
     });
     __syncthreads();
     for (int v = threadIdx.x; v < hi - lo; v += blockDim.x)
@@ -167,12 +299,15 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
   }
 }
 
-__global__ void zero_ctl_kernel(unsigned *p) { *p = 0u; }
+__global__ void zero_ctl_kernel(unsigned *p) { p[threadIdx.x] = 0u; }
+
+// Chunks drawn, then the bins' magnitudes (log_bound_kernel).
+constexpr int kCtlWords = 1 + kLogBins;
 
 int allocate(LogBuf &out) {
   LogBuf nb;
   hipError_t e = hipMalloc(&nb.rec, size_t(kLogPool) * kLogChunk * sizeof(float4));
-  if (e == hipSuccess) e = hipMalloc(&nb.ctl, sizeof(unsigned));
+  if (e == hipSuccess) e = hipMalloc(&nb.ctl, kCtlWords * sizeof(unsigned));
   if (e == hipSuccess) e = hipMalloc(&nb.meta, size_t(kLogPool) * sizeof(unsigned));
   if (e != hipSuccess) {
     (void)hipFree(nb.rec);
@@ -246,8 +381,10 @@ int log_tile() {
   int tile = 16384;
   while (tile > 1024 && size_t(tile) * sizeof(long long) + kStatic > size_t(max_lds)) tile >>= 1;
   if (tile * sizeof(long long) > 65536 &&
-      hipFuncSetAttribute(reinterpret_cast<const void *>(log_reduce_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, int(tile * sizeof(long long))) != hipSuccess) {
+      (hipFuncSetAttribute(reinterpret_cast<const void *>(log_reduce_kernel<false>),
+                           hipFuncAttributeMaxDynamicSharedMemorySize, int(tile * sizeof(long long))) != hipSuccess ||
+       hipFuncSetAttribute(reinterpret_cast<const void *>(log_reduce_kernel<true>),
+                           hipFuncAttributeMaxDynamicSharedMemorySize, int(tile * sizeof(long long))) != hipSuccess)) {
     (void)hipGetLastError();
     tile = 65536 / int(sizeof(long long)) / 2;
   }
@@ -255,11 +392,14 @@ int log_tile() {
   return tile;
 }
 
-int log_target(const Scene *s, const MediumInfo &m, float *g, LogTarget &target) {
+int log_target(const Scene *s, const MediumInfo &m, float *g, int wide, LogTarget &target) {
   const int tile = log_tile();
   const Param &P = s->params[m.sigma_param];
-  const int64_t n = int64_t(P.nx) * P.ny * P.nz;
-  if (n > int64_t(tile) * kLogMaxTiles || int64_t(P.nx) * P.ny + P.nx + 1 > tile) return 0;
+  const int64_t n = int64_t(P.nx) * P.ny * P.nz, span = int64_t(P.nx) * P.ny + P.nx + 1;
+  int extra = 0;
+  while (extra <= wide && (n > (int64_t(tile) << extra) * kLogMaxTiles || span > (int64_t(tile) << extra))) ++extra;
+  if (extra > wide) return 0;
+  target.shift = __builtin_ctz(unsigned(tile)) + extra;
   target.g = g;
   target.nx = P.nx;
   target.ny = P.ny;
@@ -273,13 +413,13 @@ int log_target(const Scene *s, const MediumInfo &m, float *g, LogTarget &target)
   return int((n + tile - 1) / tile);
 }
 
-void log_into(const LogBuf &buf, int param, unsigned bin0, GradTargets &G) {
+void log_into(const LogBuf &buf, int param, unsigned bin0, int shift, GradTargets &G) {
   G.log_rec = buf.rec;
   G.log_ctl = buf.ctl;
   G.log_meta = buf.meta;
   G.log_chunks = log_pool_chunks();
   G.log_bin0 = bin0;
-  G.log_shift = __builtin_ctz(unsigned(log_tile()));
+  G.log_shift = shift;
   G.log_param = param;
 }
 
@@ -287,10 +427,12 @@ void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunc
               int64_t samples, int64_t min_samples) {
   for (const MediumInfo &M : s->media) {
     if (M.homogeneous || M.sigma_param < 0 || !G.g[M.sigma_param]) continue;
-    log.tiles = log_target(s, M, G.g[M.sigma_param], log.target);
-    if (log.tiles > 0 && samples >= min_samples * log.tiles && stream_pool(stream, log.buf) == RCV_OK) {
-      log_into(log.buf, M.sigma_param, 0, GL);
-      hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, stream, log.buf.ctl);
+    log.tiles = log_target(s, M, G.g[M.sigma_param], kLogWide, log.target);
+    const bool wide = log.tiles > 0 && (1 << log.target.shift) > log_tile();
+    const int64_t enough = wide ? std::max(kWideLogSamples * log.tiles, kWideLogLaunch) : min_samples * log.tiles;
+    if (log.tiles > 0 && samples >= enough && stream_pool(stream, log.buf) == RCV_OK) {
+      log_into(log.buf, M.sigma_param, 0, log.target.shift, GL);
+      hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(kCtlWords), 0, stream, log.buf.ctl);
     } else {
       log.target.g = nullptr;
     }
@@ -301,13 +443,25 @@ void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunc
 void reduce_log(const LogLaunch &log, const GradTargets &GL, hipStream_t stream) {
   if (!log.target.g) return;
   const int tile = log_tile();
-  hipLaunchKernelGGL(log_reduce_kernel, dim3(kLogSplits, log.tiles), dim3(kReduceBlock),
-                     size_t(tile) * sizeof(long long), stream, log.buf.rec, log.buf.ctl, log.buf.meta, GL.log_chunks,
-                     log.target, static_cast<const LogTarget *>(nullptr), 1, tile);
+  // about 2048 blocks
+  const dim3 grid(std::min(kLogSplits, std::max(kLogMinSplits, 2048 / log.tiles)), log.tiles);
+  const LogBuf &L = log.buf;
+  const size_t lds = size_t(tile) * sizeof(long long);
+  const LogTarget *const none = nullptr;
+  if ((1 << log.target.shift) > tile) {
+    unsigned *const bound = L.ctl + 1;
+    hipLaunchKernelGGL(log_bound_kernel, dim3(kBoundBlocks), dim3(kBoundBlock), 0, stream, L.rec, L.ctl, L.meta,
+                       GL.log_chunks, bound);
+    hipLaunchKernelGGL(log_reduce_kernel<true>, grid, dim3(kReduceBlock), lds, stream, L.rec, L.ctl, L.meta,
+                       GL.log_chunks, log.target, none, 1, tile, bound);
+  } else {
+    hipLaunchKernelGGL(log_reduce_kernel<false>, grid, dim3(kReduceBlock), lds, stream, L.rec, L.ctl, L.meta,
+                       GL.log_chunks, log.target, none, 1, tile, static_cast<const unsigned *>(nullptr));
+  }
 }
 
 void zero_log(const LogBuf &buf, hipStream_t stream) {
-  hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(1), 0, stream, buf.ctl);
+  hipLaunchKernelGGL(zero_ctl_kernel, dim3(1), dim3(kCtlWords), 0, stream, buf.ctl);
 }
 
 void reduce_log_batch(const LogBuf &buf, const LogTarget &first, const LogTarget *targets, int n, int tiles,
@@ -315,8 +469,9 @@ void reduce_log_batch(const LogBuf &buf, const LogTarget &first, const LogTarget
   const int tile = log_tile();
   // about 4096 blocks
   const int splits = std::min(kLogSplits, std::max(4, 4096 / tiles));
-  hipLaunchKernelGGL(log_reduce_kernel, dim3(splits, tiles), dim3(kReduceBlock), size_t(tile) * sizeof(long long),
-                     stream, buf.rec, buf.ctl, buf.meta, log_pool_chunks(), first, targets, n, tile);
+  hipLaunchKernelGGL(log_reduce_kernel<false>, dim3(splits, tiles), dim3(kReduceBlock), size_t(tile) * sizeof(long long),
+                     stream, buf.rec, buf.ctl, buf.meta, log_pool_chunks(), first, targets, n, tile,
+                     static_cast<const unsigned *>(nullptr));
 }
 
 bool take_log_pool(LogBuf &buf) {

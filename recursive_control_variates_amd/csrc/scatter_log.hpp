@@ -13,7 +13,7 @@ constexpr unsigned kLogPool = 786432;
 
 struct LogBuf {
   float4 *rec = nullptr;
-  unsigned *ctl = nullptr;   // chunks drawn
+  unsigned *ctl = nullptr;   // chunks drawn, bins' magnitudes
   unsigned *meta = nullptr;  // kLogPool chunk bins and record counts
 };
 
@@ -28,20 +28,37 @@ struct LogLaunch {
 // Voxels per reduction tile on the current device.
 int log_tile();
 
-// Whether the density gradient `g` of medium m of scene s can be logged (its
-// grid fits the reduction tiles and a footprint spans at most two of them);
-// fills target's grid and returns its tiles, or 0.
-int log_target(const Scene *s, const MediumInfo &m, float *g, LogTarget &target);
+// Reduction tiles per bin of a large grid's log, as a power of two, at most
+// (every tile of a bin reads the bin's records), and the samples per tile and
+// in all from which a launch on such a grid is logged: below them the
+// reduction's cost per tile, and the chunks its wavefronts leave nearly empty,
+// weigh more than the atomics, which a launch that does not fill the device
+// hides behind its longest path. Adjoint call with atomics / logged, one
+// view, optical depth ~3: 80^3 (32 tiles) with 128 Ki samples 1.01 / 1.09 ms,
+// 256 Ki 1.03 / 1.08, 512 Ki 1.64 / 1.35; 100^3 (62) with 512 Ki 1.63 / 1.57,
+// 1 Mi 3.04 / 2.26; 128^3 (128) with 512 Ki 1.70 / 1.90, 1 Mi 3.09 / 2.76,
+// 2 Mi 5.45 / 3.99; 150^3 (206) with 2 Mi 5.39 / 5.09. Optical depth ~15:
+// 80^3 with 512 Ki 12.3 / 3.7 ms, 128^3 with 1 Mi 24.9 / 10.8.
+constexpr int kLogWide = 4;
+constexpr int64_t kWideLogSamples = 8192;
+constexpr int64_t kWideLogLaunch = int64_t(1) << 19;
 
-// Points G at the pool for gradient `param` with chunk bins from bin0 on.
-void log_into(const LogBuf &buf, int param, unsigned bin0, GradTargets &G);
+// Whether the density gradient `g` of medium m of scene s can be logged with
+// bins of up to 2^wide reduction tiles (its grid fits the bins and a footprint
+// spans at most two of them); fills target's grid and returns its tiles, or 0.
+int log_target(const Scene *s, const MediumInfo &m, float *g, int wide, LogTarget &target);
+
+// Points G at the pool for gradient `param` with chunk bins of 2^shift voxels
+// from bin0 on.
+void log_into(const LogBuf &buf, int param, unsigned bin0, int shift, GradTargets &G);
 
 // Sets up the log of a launch on `stream` for the density gradient of the
 // first heterogeneous medium that has one, with the stream's pool. Without
-// memory for it, or with fewer than `min_samples` (per reduction tile) of the
-// launch's `samples`, the scatter-adds stay atomics.
+// memory for it, or with fewer of the launch's `samples` than the bins ask for
+// (kWideLogSamples; `min_samples` per tile for bins of one tile), the
+// scatter-adds stay atomics.
 void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL,
-              int64_t samples = 0, int64_t min_samples = 0);
+              int64_t samples, int64_t min_samples = 0);
 
 // Adds the records of a launch to its gradient.
 void reduce_log(const LogLaunch &log, const GradTargets &GL, hipStream_t stream);

@@ -520,12 +520,10 @@ struct GridFoot {
 // the point where the scatter log is added up.)
 __device__ inline float voxel_coord(float l, int n) { return __builtin_fmaf(l, float(n), -0.5f); }
 
-// (P: a ParamBind or LogTarget; M: a MediumInfo or LogTarget)
-template <class Grid, class Box>
-__device__ inline void grid_footprint(const Grid &P, const Box &M, V3 p, GridFoot &g) {
-  const float lx = (p.x - M.lo[0]) / (M.hi[0] - M.lo[0]);
-  const float ly = (p.y - M.lo[1]) / (M.hi[1] - M.lo[1]);
-  const float lz = (p.z - M.lo[2]) / (M.hi[2] - M.lo[2]);
+// The footprint at relative position (lx, ly, lz) of the grid's box (P: a
+// ParamBind or LogTarget).
+template <class Grid>
+__device__ inline void grid_footprint_at(const Grid &P, float lx, float ly, float lz, GridFoot &g) {
   const float x = voxel_coord(lx, P.nx), y = voxel_coord(ly, P.ny), z = voxel_coord(lz, P.nz);
   const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
   g.tx = x - fx;
@@ -539,6 +537,15 @@ __device__ inline void grid_footprint(const Grid &P, const Box &M, V3 p, GridFoo
   g.dx = x1 - x0;
   g.dy = (y1 - y0) * P.nx;
   g.dz = (z1 - z0) * P.nx * P.ny;
+}
+
+// (M: a MediumInfo or LogTarget)
+template <class Grid, class Box>
+__device__ inline void grid_footprint(const Grid &P, const Box &M, V3 p, GridFoot &g) {
+  const float lx = (p.x - M.lo[0]) / (M.hi[0] - M.lo[0]);
+  const float ly = (p.y - M.lo[1]) / (M.hi[1] - M.lo[1]);
+  const float lz = (p.z - M.lo[2]) / (M.hi[2] - M.lo[2]);
+  grid_footprint_at(P, lx, ly, lz, g);
 }
 
 __device__ inline float grid_eval1(const float *data, const GridFoot &g) {

@@ -23,9 +23,11 @@
 
 namespace rcv {
 
-// Scatter log geometry: reduction tiles of a logged gradient, bins (one per
-// tile, then one per seam between tiles t and t + 1; the last seam does not
-// exist), records per chunk, chunks a wavefront draws from the pool at once.
+// Scatter log geometry: ranges of voxels a logged gradient is split into, bins
+// (one per range, then one per seam between ranges t and t + 1; the last seam
+// does not exist), records per chunk, chunks a wavefront draws from the pool
+// at once. A range is a reduction tile or, for a larger grid, a power of two
+// of them.
 constexpr int kLogMaxTiles = 16;
 constexpr int kLogBins = 2 * kLogMaxTiles;
 constexpr unsigned kLogChunk = 256;
@@ -37,9 +39,9 @@ struct GradTargets {
   float *g[kMaxParams];
   // Scatter log (the persistent volume adjoints): the replay pass appends
   // each scatter-add into g[log_param] as a record (point, value) in log_rec
-  // instead of adding it. Records are binned by the reduction tile
-  // (2^log_shift voxels) their corners fall in: bin t for tile t, bin
-  // kLogMaxTiles + t for footprints across tiles t and t + 1. A wavefront
+  // instead of adding it. Records are binned by the range of 2^log_shift
+  // voxels their corners fall in: bin t for range t, bin kLogMaxTiles + t for
+  // footprints across ranges t and t + 1. A wavefront
   // fills chunks of kLogChunk records, one per bin at a time, drawn kLogDraw
   // at a time from a pool of log_chunks: *log_ctl counts the chunks drawn,
   // log_meta[c] holds chunk c's bin (log_bin0 + bin, so that several
@@ -69,14 +71,15 @@ struct GradTargets {
 
 // A gradient whose scatter-adds are logged, for the reduction: the grid, its
 // placement (footprints are formed again from the records' points), the
-// first bin of its chunks and the first of its tiles among those of all
-// gradients of the launch.
+// first bin of its chunks, the first of its tiles among those of all
+// gradients of the launch and the log2 of its bins' voxels.
 struct LogTarget {
   float *g;
   int nx, ny, nz;
   float lo[3], hi[3];
   unsigned bin0;
   int tile0;
+  int shift;
 };
 
 // Event counters of a launch (scene counting mode): each call adds n per

@@ -433,3 +433,45 @@ def test_texture_adjoint_matches_oracle_same_samples(cuda):
                       integrator_type=0)
     assert g_gpu.shape == g_cpu.shape == (16, 16, 3)
     _close_to_oracle(g_gpu, g_cpu)
+
+
+# Bins of two and of eight reduction tiles; slices larger than a tile (a
+# footprint spans three of them); a pool that runs out; a NaN image gradient.
+@pytest.mark.parametrize("shape,kind,chunks,nan", [
+    ((64, 72, 72), "prbvolpath", None, False),
+    ((33, 200, 170), "prbvolpath", None, False),
+    ((64, 72, 72), "volpathsimple", None, False),
+    ((64, 72, 72), "prbvolpath", "40", False),
+    ((64, 72, 72), "prbvolpath", None, True),
+])
+def test_scatter_log_of_large_grids_equals_atomics(cuda, monkeypatch, shape, kind, chunks, nan):
+    # Grids of more than 16 reduction tiles are logged from 2^19 samples on
+    # (and 8192 a tile; 819200 here), against the static launch's atomics on
+    # the same samples. A voxel gets some 10^3 terms at most, whose float sums
+    # in two orders differ by ~sqrt(10^3) 2^-24 = 2e-6 of the largest partial
+    # sum; ten times that for partial sums above the result.
+    announce(f"scatter log of a large grid {shape} {kind} pool {chunks} nan {nan}")
+    if chunks:
+        monkeypatch.setenv("RCV_SCATTER_LOG_CHUNKS", chunks)
+    rng = np.random.default_rng(29)
+    grid = (0.2 + rng.uniform(0, 0.8, shape + (1,))).astype(np.float32)
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=0.8, scale=5.0, w=160, h=160, spp=32))
+    gimg = rng.uniform(0.5, 1.5, (160, 160, 3)).astype(np.float32)
+    if nan:
+        gimg[80, 80] = np.nan
+    gimg = torch.from_numpy(gimg).cuda()
+    integ = rcv.load_dict({"type": kind, "max_depth": 8, "rr_depth": 8})
+    p = rcv.traverse(sc)
+    p[KEY] = p[KEY].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    grads = []
+    for spt in (0, 4):
+        integ.samples_per_thread = spt
+        grads.append(integ.adjoint(sc, p, gimg, 0, 61, 32)[KEY].double().cpu().numpy())
+    a, b = grads
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.isnan(b).any() == nan
+    a, b = a[~np.isnan(a)], b[~np.isnan(b)]
+    scale = np.abs(b).max()
+    assert scale > 0 and (b != 0).mean() > 0.5, (b != 0).mean()
+    assert np.allclose(a, b, rtol=1e-4, atol=2e-5 * scale), np.abs(a - b).max() / scale
