@@ -221,3 +221,33 @@ def test_one_box_adjoint_equals_general(cuda, shape, factor, albedo, scale, dept
         scale_g = np.abs(b).max()
         assert scale_g > 0
         assert np.allclose(a, b, rtol=1e-4, atol=1e-4 * scale_g), np.abs(a - b).max() / scale_g
+
+
+@pytest.mark.parametrize("kind", ["prbvolpath", "volpathsimple"])
+def test_captured_adjoint_replays(cuda, kind):
+    # A capture may be the first launch of its stream: the scatter log's pool
+    # is not allocated then. The graph is replayed several times with eager
+    # work between; a voxel's few hundred terms differ by their order only
+    # (2e-5 of the largest gradient, as above).
+    announce(f"captured adjoint ({kind})")
+    rng = np.random.default_rng(59)
+    grid = (0.2 + rng.uniform(0, 0.8, (20, 20, 20, 1))).astype(np.float32)
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=0.8, scale=5.0, w=48, h=32, spp=16))
+    gimg = torch.from_numpy(rng.uniform(0.5, 1.5, (32, 48, 3)).astype(np.float32)).cuda()
+    integ = rcv.load_dict({"type": kind, "max_depth": 8, "rr_depth": 4})
+    p = rcv.traverse(sc)
+    p[KEY] = p[KEY].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    ref = integ.adjoint(sc, p, gimg, 0, 67, 16)[KEY].double().cpu().numpy()
+    scale = np.abs(ref).max()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        out = integ.adjoint(sc, p, gimg, 0, 67, 16)[KEY]
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.double().cpu().numpy()
+        assert np.allclose(got, ref, rtol=1e-4, atol=2e-5 * scale), np.abs(got - ref).max() / scale
+        integ.adjoint(sc, p, gimg, 0, 71, 16)
+        torch.cuda.synchronize()
