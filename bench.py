@@ -313,11 +313,11 @@ def rooflines(run, counts, window):
     first, count = window
     out = {}
     kinds = [("volume_adjoint", "adj_ms", "adjoint_bytes",
-              "adjoint_persistent_kernel<VOLPATH> + log_reduce_kernel (path replay and its scatter-log "
+              "box_kernel<1, adjoint> + log_reduce_kernel (path replay and its scatter-log "
               "reduction, one rcv_render_backward call)")]
     if run["ts_ms"] is not None:
         kinds.append(("volume_twostate", "ts_ms", "twostate_bytes",
-                      "render_persistent_kernel<2, VOLPATH> (two-state delta tracking)"))
+                      "box_kernel<2, render> (two-state delta tracking)"))
     for name, mkey, bkey, kern in kinds:
         ms = np.array([run[mkey][i] for i in idx])
         by = np.array([counts[i][bkey] for i in idx], np.float64)
