@@ -393,6 +393,10 @@ int log_tile() {
 }
 
 int log_target(const Scene *s, const MediumInfo &m, float *g, int wide, LogTarget &target) {
+  for (const MediumInfo &o : s->media)
+    if (!o.homogeneous && o.sigma_param == m.sigma_param &&
+        !(std::equal(o.lo, o.lo + 3, m.lo) && std::equal(o.hi, o.hi + 3, m.hi)))
+      return 0;
   const int tile = log_tile();
   const Param &P = s->params[m.sigma_param];
   const int64_t n = int64_t(P.nx) * P.ny * P.nz, span = int64_t(P.nx) * P.ny + P.nx + 1;

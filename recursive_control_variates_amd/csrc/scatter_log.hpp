@@ -45,7 +45,9 @@ constexpr int64_t kWideLogLaunch = int64_t(1) << 19;
 
 // Whether the density gradient `g` of medium m of scene s can be logged with
 // bins of up to 2^wide reduction tiles (its grid fits the bins and a footprint
-// spans at most two of them); fills target's grid and returns its tiles, or 0.
+// spans at most two of them, and every medium over the grid places it alike: a
+// record holds its world point, from which the reduction forms the footprint
+// with the target's one box); fills target's grid and returns its tiles, or 0.
 int log_target(const Scene *s, const MediumInfo &m, float *g, int wide, LogTarget &target);
 
 // Points G at the pool for gradient `param` with chunk bins of 2^shift voxels
