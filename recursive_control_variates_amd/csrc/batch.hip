@@ -49,6 +49,13 @@ __device__ inline uint32_t float_key_dev(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// The states of a one-box job's tracker: those of its view, whose optimised
+// parameter is the ring's whatever the scene has bound.
+__host__ __device__ inline void bind_box(BatchJobDev &J) {
+  J.box.sigma = J.view.params[J.box.med.sigma_param];
+  if (J.box.med.albedo_param >= 0) J.box.albedo = J.view.params[J.box.med.albedo_param];
+}
+
 // ---------------------------------------------------------------- 1. rotate
 __global__ void batch_rotate_kernel(BatchJobDev *jobs, int n_jobs, unsigned *queues) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -66,10 +73,7 @@ __global__ void batch_rotate_kernel(BatchJobDev *jobs, int n_jobs, unsigned *que
     J.view.params[J.param].data[RCV_STATE_NEW] = J.ring[J.ring_new];
     J.maj_keys[RCV_STATE_OLD] = J.maj_keys[RCV_STATE_NEW];
     J.maj_keys[RCV_STATE_NEW] = J.next_key;
-    if (J.box_queue) {
-      J.box.sigma = J.view.params[J.box.med.sigma_param];
-      if (J.box.med.albedo_param >= 0) J.box.albedo = J.view.params[J.box.med.albedo_param];
-    }
+    if (J.box_queue) bind_box(J);
   }
   J.next_key = float_key_dev(-kInf);
 }
@@ -507,7 +511,10 @@ extern "C" int rcv_batch_add_job(rcv_batch *b, const rcv_batch_job *d, int32_t *
   J.box_queue = nullptr;
   J.box_partial = nullptr;
   const bool box = takes_box(s, &d->integrator);
-  if (box) J.box = bound_box(s);
+  if (box) {
+    J.box = bound_box(s);
+    bind_box(J);
+  }
   b->is_box.push_back(box);
   if (J.itype == RCV_INTEGRATOR_VOLPATH && !box) b->feat |= s->features();
   b->host_jobs.push_back(J);
