@@ -12,9 +12,15 @@
  *   - `stream` is a hipStream_t passed as void* (NULL = legacy default stream).
  *     All device work is enqueued on it; no call synchronises the host unless
  *     stated.
- *   - Scene handles are thread-compatible (one thread at a time); a CV state is
- *     not re-entrant: two rcv_cv_step calls on one state must be ordered on one
- *     stream.
+ *   - Scene handles are thread-compatible (one thread at a time). Calls on one
+ *     scene may overlap on several streams: each stream has its own launch
+ *     scratch (96 bytes per pixel of the largest sensor, for a small image of a
+ *     medium in a box more, 6 MB at most; allocated at its first call, kept
+ *     until the scene is destroyed; past 32 streams a new one waits for the
+ *     device and takes over another's). Captured launches of a scene share one more: graphs that
+ *     hold renders or adjoints of one scene must not run at the same time.
+ *   - A CV state is not re-entrant: two rcv_cv_step calls on one state must be
+ *     ordered on one stream.
  *   - Images are row-major (height, width, 3) float32. Textures are
  *     (height, width, channels); grids are (depth, height, width, channels).
  */

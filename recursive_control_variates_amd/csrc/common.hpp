@@ -50,6 +50,18 @@ inline int check_launch(const char *name) {
     if (!(cond)) return ::rcv::fail(RCV_E_INVALID, __VA_ARGS__); \
   } while (0)
 
+// Whether `stream` is being captured into a graph (the legacy default stream
+// cannot be). True when that cannot be told.
+inline bool capturing(hipStream_t stream) {
+  if (!stream) return false;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 inline bool aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

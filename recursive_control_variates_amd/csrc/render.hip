@@ -586,24 +586,33 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
   const unsigned grid = ceil_div(threads, block);
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
   const RenderLaunch L{dim3(grid), block, stream, &s->view, I, sensor, seed, spp, spt, cl2, img_old, img_new};
-  if (takes_box(s, d)) {
+  // under capture, launches that would be static without the tracker stay so:
+  // several graphs of a scene share its scratch
+  const bool captured = capturing(stream);
+  const bool few_units = (1 << cl2) <= kRenderMaxUnitsPerPixel;
+  const bool box = takes_box(s, d) && (!captured || few_units);
+  const bool persistent = d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && few_units;
+  LaunchScratch tmp;
+  if (box || persistent)
+    if (int rc = s->scratch(stream, captured, tmp)) return rc;
+  if (box) {
     const int ucl2 = box_chunk_log2(s, n_pix, spp, cl2, 3 * ns);
     const GradTargets none = no_targets();
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
     launch_box(s, ns, kBoxRender,
                BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), nullptr, &none,
-                         s->partial, s->work_queue});
+                         tmp.partial, tmp.queue});
     if (ns == 2)
-      hipLaunchKernelGGL(reduce_units_kernel<2>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+      hipLaunchKernelGGL(reduce_units_kernel<2>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, tmp.partial, n_pix,
                          ucl2, spp, img_old, img_new);
     else
-      hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+      hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, tmp.partial, n_pix,
                          ucl2, spp, img_old, img_new);
   } else if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE) {
     with_volume_features(s->features(), [&](auto f) {
       launch_render_kernel<1, RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>(L);
     });
-  } else if (d->type == RCV_INTEGRATOR_VOLPATH && !d->samples_per_thread && (1 << cl2) <= kRenderMaxUnitsPerPixel) {
+  } else if (persistent) {
     // persistent, with at most kRenderMaxUnitsPerPixel units per pixel (the
     // unit-sum buffer); smaller images that need more units per pixel to
     // fill the device take the static launch below
@@ -611,19 +620,19 @@ int launch_render(const Scene *s, const rcv_integrator_desc *d, int sensor, uint
     while ((2 << ucl2) <= kRenderMaxUnitsPerPixel && (spp >> (ucl2 + 1)) >= kVolUnitSamples) ++ucl2;
     const unsigned units = unsigned(n_pix << ucl2);
     RCV_REQUIRE(int64_t(units) * 3 * ns <= s->partial_cap, "%s: unit buffer too small", fn);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
     auto go = [&](auto kern) {
       const unsigned pgrid = std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)), grid);
       hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
-                         ucl2, s->partial, s->work_queue, units);
+                         ucl2, tmp.partial, tmp.queue, units);
     };
     if (ns == 2) {
       with_render_features(s->features(), [&](auto f) { go(render_persistent_kernel<2, decltype(f)::value>); });
-      hipLaunchKernelGGL(reduce_units_kernel<2>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+      hipLaunchKernelGGL(reduce_units_kernel<2>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, tmp.partial, n_pix,
                          ucl2, spp, img_old, img_new);
     } else {
       with_render_features(s->features(), [&](auto f) { go(render_persistent_kernel<1, decltype(f)::value>); });
-      hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+      hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, tmp.partial, n_pix,
                          ucl2, spp, img_old, img_new);
     }
   } else if (d->type == RCV_INTEGRATOR_VOLPATH) {
@@ -671,6 +680,9 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
   const int block = d->block_size ? d->block_size : kDefaultBlock;
   const unsigned grid = ceil_div(n_pix << cl2, block);
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
+  LaunchScratch tmp;
+  if (!d->samples_per_thread)
+    if (int rc = s->scratch(stream, capturing(stream), tmp)) return rc;
   // the per-sample integrators' persistent adjoint, as the volume path
   // tracer's below
   auto launch_sample_persistent = [&](auto kern, const GradTargets &targets) {
@@ -678,9 +690,9 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     const unsigned units = unsigned(n_pix << ucl2);
     const unsigned pgrid =
         std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)), ceil_div(int64_t(units), block));
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
     hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp, ucl2,
-                       grad_img, targets, s->work_queue, units);
+                       grad_img, targets, tmp.queue, units);
   };
   if (d->type == RCV_INTEGRATOR_VOLPATH_SIMPLE && !d->samples_per_thread) {
     GradTargets GL = G;
@@ -688,9 +700,9 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     open_log(s, G, stream, log, GL, n_pix * spp, kSimpleLogSamples);
     if (takes_simple_box(s, d)) {
       const int ucl2 = unit_chunk_log2(spp, cl2, kVolUnitSamples);
-      hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+      hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
       launch_simple_box(s, BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), grad_img, &GL,
-                                     nullptr, s->work_queue});
+                                     nullptr, tmp.queue});
     } else {
       with_volume_features(s->features(), [&](auto f) {
         launch_sample_persistent(adjoint_sample_persistent_kernel<RCV_INTEGRATOR_VOLPATH_SIMPLE, decltype(f)::value>,
@@ -721,10 +733,10 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
         GL.hom_once = false;
     LogLaunch log;
     if (!taped) open_log(s, G, stream, log, GL, n_pix * spp);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
     if (box)
       launch_box(s, 1, kBoxAdjoint,
-                 BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, units, grad_img, &GL, nullptr, s->work_queue});
+                 BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, units, grad_img, &GL, nullptr, tmp.queue});
     else
       with_render_features(s->features(), [&](auto f) {
         // the waves that fit, pulling units of >= kVolUnitSamples samples
@@ -734,7 +746,7 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
           const unsigned pgrid = std::min(resident_grid(reinterpret_cast<const void *>(kern), block, stack_bytes(block)),
                                           ceil_div(int64_t(units), block));
           hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
-                             ucl2, grad_img, GL, s->work_queue, units);
+                             ucl2, grad_img, GL, tmp.queue, units);
         };
         // three waves per SIMD with the log or without scatter-adds, four
         // with atomics (kWavesPerEuLoggedAdjoint)
@@ -790,13 +802,16 @@ int launch_forward(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
   const int block = d->block_size ? d->block_size : kDefaultBlock;
   const unsigned grid = ceil_div(n_pix << cl2, block);
   if (s->view.counters) hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, stream, s->view.counters);
-  if (takes_box(s, d)) {
+  // (captured: the static launch, which needs no scratch)
+  if (takes_box(s, d) && !capturing(stream)) {
+    LaunchScratch tmp;
+    if (int rc = s->scratch(stream, false, tmp)) return rc;
     const int ucl2 = box_chunk_log2(s, n_pix, spp, cl2, 3);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, s->work_queue);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
     launch_box(s, 1, kBoxForward,
-               BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), nullptr, &T, s->partial,
-                         s->work_queue});
-    hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, s->partial, n_pix,
+               BoxLaunch{stream, block, I, sensor, seed, spp, ucl2, unsigned(n_pix << ucl2), nullptr, &T, tmp.partial,
+                         tmp.queue});
+    hipLaunchKernelGGL(reduce_units_kernel<1>, dim3(ceil_div(n_pix, 256)), dim3(256), 0, stream, tmp.partial, n_pix,
                        ucl2, spp, nullptr, dimg);
   } else if (d->type == RCV_INTEGRATOR_VOLPATH)
     with_render_features(s->features(), [&](auto f) {

@@ -443,8 +443,6 @@ int Scene::upload(hipStream_t stream) {
   const size_t o_maj = put(maj_init.data(), maj_init.size() * 4);
   std::vector<unsigned long long> cnt(kNumCounters, 0ull);
   const size_t o_cnt = put(cnt.data(), cnt.size() * 8);
-  const unsigned q_init[4] = {0u, 0u, 0u, 0u};
-  const size_t o_q = put(q_init, sizeof(q_init));
 
   RCV_TRY_HIP(hipMalloc(&dev_block, blob.size()), "rcv_scene_commit: hipMalloc");
   // the scenes of the one-box tracker
@@ -459,8 +457,8 @@ int Scene::upload(hipStream_t stream) {
     int64_t max_pix = 0;
     for (auto &sen : sensors) max_pix = std::max(max_pix, int64_t(sen.film_w) * sen.film_h);
     partial_cap = std::max(max_pix * kRenderMaxUnitsPerPixel, one_box ? std::min(max_pix * 64, kRenderMinUnits) : 0) * 6;
-    if (partial_cap > 0)
-      RCV_TRY_HIP(hipMalloc(&partial, size_t(partial_cap) * sizeof(float)), "rcv_scene_commit: hipMalloc");
+    // (the first stream's)
+    if (int rc = add_scratch(nullptr, false)) return rc;
   }
   RCV_TRY_HIP(hipMemcpyAsync(dev_block, blob.data(), blob.size(), hipMemcpyHostToDevice, stream),
               "rcv_scene_commit: upload");
@@ -486,7 +484,6 @@ int Scene::upload(hipStream_t stream) {
   majorant_keys = reinterpret_cast<uint32_t *>(base + o_maj);
   v.majorants = reinterpret_cast<const float *>(majorant_keys);
   counters = reinterpret_cast<unsigned long long *>(base + o_cnt);
-  work_queue = reinterpret_cast<unsigned *>(base + o_q);
   v.counters = nullptr;
   v.flat = reinterpret_cast<const FlatPrim *>(base + o_flat);
   v.n_flat = int(flat.size());
@@ -546,6 +543,50 @@ int Scene::upload(hipStream_t stream) {
         int rc = reduce_param(i, s, stream);
         if (rc != RCV_OK) return rc;
       }
+  return RCV_OK;
+}
+
+int Scene::add_scratch(hipStream_t stream, bool captured) const {
+  // an allocation breaks off captures of its thread, unless it is told not to mind them
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RCV_TRY_HIP(hipThreadExchangeStreamCaptureMode(&mode), "launch scratch: capture mode");
+  void *p = nullptr;
+  const size_t sums = size_t(partial_cap) * sizeof(float);
+  const hipError_t e = hipMalloc(&p, sums + 256);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return hip_fail(e, "launch scratch: hipMalloc");
+  }
+  LaunchScratch mem;
+  mem.partial = static_cast<float *>(p);
+  mem.queue = reinterpret_cast<unsigned *>(static_cast<char *>(p) + sums);
+  scratches.push_back(OwnedScratch{mem, stream, captured, 0});
+  return RCV_OK;
+}
+
+int Scene::scratch(hipStream_t stream, bool captured, LaunchScratch &out) const {
+  OwnedScratch *own = nullptr, *oldest = nullptr;
+  int streams = 0;
+  for (OwnedScratch &o : scratches) {
+    if (o.captured != captured) continue;
+    if (captured || (o.used && o.stream == stream)) own = &o;
+    if (!captured) {
+      ++streams;
+      if (!oldest || o.used < oldest->used) oldest = &o;
+    }
+  }
+  if (!own && oldest && (!oldest->used || streams >= kMaxScratchStreams)) {
+    if (oldest->used) RCV_TRY_HIP(hipDeviceSynchronize(), "launch scratch: synchronize");
+    oldest->stream = stream;
+    own = oldest;
+  }
+  if (!own) {
+    if (int rc = add_scratch(stream, captured)) return rc;
+    own = &scratches.back();
+  }
+  own->used = ++scratch_uses;
+  out = own->mem;
   return RCV_OK;
 }
 
@@ -659,7 +700,7 @@ bool Scene::box_path() const {
 Scene::~Scene() {
   if (dev_block) (void)hipFree(dev_block);
   if (sg_block) (void)hipFree(sg_block);
-  if (partial) (void)hipFree(partial);
+  for (const OwnedScratch &o : scratches) (void)hipFree(o.mem.partial);
 }
 
 }  // namespace rcv

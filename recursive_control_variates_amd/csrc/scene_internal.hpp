@@ -26,6 +26,19 @@ struct Param {
   const float *data[2] = {nullptr, nullptr};
 };
 
+// What a persistent launch needs beside its arguments: the counter its lanes
+// draw work units from and, for renders and forward mode, the units' sums
+// (Scene::partial_cap floats). One per stream that a scene is used on, so that
+// launches on different streams may overlap, and one for the launches of
+// captured graphs, which run on whatever stream replays them.
+struct LaunchScratch {
+  unsigned *queue = nullptr;
+  float *partial = nullptr;
+};
+// Streams with a scratch of their own, at most: another one takes over the
+// scratch that was used longest ago, once the device is idle.
+constexpr int kMaxScratchStreams = 32;
+
 struct Scene {
   // collected before commit
   std::vector<Param> params;
@@ -52,9 +65,15 @@ struct Scene {
   MediumInfo *media_dev = nullptr;  // device copy of `media`
   int batch_refs = 0;               // batches holding this scene (no relayout then)
   unsigned long long *counters = nullptr;
-  unsigned *work_queue = nullptr;  // unit counter of the persistent launches
-  float *partial = nullptr;        // per work unit radiance sums of a persistent render
-  int64_t partial_cap = 0;         // floats
+  int64_t partial_cap = 0;          // floats of a LaunchScratch's unit sums
+  struct OwnedScratch {
+    LaunchScratch mem;
+    hipStream_t stream;  // of eager launches
+    bool captured;       // of captured launches
+    uint64_t used;       // 0: not used yet
+  };
+  mutable std::vector<OwnedScratch> scratches;
+  mutable uint64_t scratch_uses = 0;
   int n_nodes = 0;
   float bs_center[3] = {0, 0, 0};
   float bs_radius = 0;
@@ -68,6 +87,9 @@ struct Scene {
   ~Scene();
 
   int upload(hipStream_t stream);
+  // The scratch of eager launches on `stream`, or of captured ones.
+  int scratch(hipStream_t stream, bool captured, LaunchScratch &out) const;
+  int add_scratch(hipStream_t stream, bool captured) const;
   int reduce_param(int param, int state, hipStream_t stream);
   int build_supergrid(int medium, int state, hipStream_t stream);
   int64_t plan_supergrids();
