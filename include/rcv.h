@@ -214,8 +214,7 @@ int rcv_render_twostates(const rcv_scene *scene,
  * volume integrators' adjoints (samples_per_thread 0) log density
  * scatter-adds in a buffer that the library allocates on first use per
  * (device, stream), about 3.3 GB, and keeps until the process ends; calls on
- * one stream share it in stream order. A first call while the stream is being
- * captured allocates nothing and adds with atomics. */
+ * one stream share it in stream order. A captured call adds with atomics. */
 int rcv_render_backward(const rcv_scene *scene,
                         const rcv_integrator_desc *integrator, int32_t sensor,
                         uint32_t seed, int32_t spp, const float *grad_img,

@@ -322,9 +322,10 @@ int allocate(LogBuf &out) {
 
 // The pool of single launches: one per (device, stream), kept for the
 // process (launches on one stream run in order; other streams get their own).
-// None is allocated while the stream is being captured, which an allocation
-// would break off: a launch captured before any other has no log.
+// A captured launch has none: its graph is replayed on any stream, beside
+// launches that log into the pool of the capture's.
 int stream_pool(hipStream_t stream, LogBuf &out) {
+  if (capturing(stream)) return 1;
   static std::mutex mu;
   static std::map<std::pair<int, hipStream_t>, LogBuf> bufs;
   int dev = 0;
@@ -333,12 +334,6 @@ int stream_pool(hipStream_t stream, LogBuf &out) {
   const auto key = std::make_pair(dev, stream);
   auto it = bufs.find(key);
   if (it == bufs.end()) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
-      (void)hipGetLastError();
-      return 1;
-    }
-    if (capture != hipStreamCaptureStatusNone) return 1;
     LogBuf nb;
     if (int rc = allocate(nb)) return rc;
     it = bufs.emplace(key, nb).first;

@@ -56,7 +56,7 @@ void log_into(const LogBuf &buf, int param, unsigned bin0, int shift, GradTarget
 
 // Sets up the log of a launch on `stream` for the density gradient of the
 // first heterogeneous medium that has one, with the stream's pool. Without
-// memory for it, or with fewer of the launch's `samples` than the bins ask for
+// memory for it, under capture, or with fewer of the launch's `samples` than the bins ask for
 // (kWideLogSamples; `min_samples` per tile for bins of one tile), the
 // scatter-adds stay atomics.
 void open_log(const Scene *s, const GradTargets &G, hipStream_t stream, LogLaunch &log, GradTargets &GL,

@@ -117,3 +117,32 @@ def test_replays_beside_eager_calls(cuda, name, w, h):
         _assert_close(name, out, want[0])
         _assert_close(name, beside, want[1])
         _assert_close(name, here, want[2])
+
+
+@pytest.mark.parametrize("kind", ["prbvolpath", "volpathsimple"])
+def test_captured_adjoint_after_an_eager_one(cuda, kind):
+    # The capture's stream has its scatter log from an eager call before; the
+    # graph is replayed on another stream while eager adjoints log on that one,
+    # of another scene with larger sums.
+    announce(f"captured {kind} adjoint after an eager one on its stream, replayed beside others")
+    name = "adjoint" if kind == "prbvolpath" else "volpathsimple adjoint"
+    (a, b) = (_scene(), _scene())
+    b[3].mul_(50.0)
+    call, other = _calls(*a)[name], _calls(*b)[name]
+    want, want_other = call(400), other(401)
+    torch.cuda.synchronize()
+    side, replays = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        call(402)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = call(400)
+    for _ in range(4):
+        with torch.cuda.stream(replays):
+            graph.replay()
+        with torch.cuda.stream(side):
+            beside = other(401)
+        torch.cuda.synchronize()
+        _assert_close(name, out, want)
+        _assert_close(name, beside, want_other)
