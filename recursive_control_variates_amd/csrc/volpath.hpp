@@ -943,6 +943,9 @@ struct VolPath {
   __device__ bool end_adjoint(const SceneView &S, LocalCounters &cnt, const GradTargets *G) {
     if constexpr (kHomOnce) {
       if (G->hom_once) {
+        // (a path without radiance may hold infinite coefficients: a medium
+        // of extinction 0 left towards infinity)
+        if (!any_nonzero(L[0])) return true;
         hom.s += float(double(dot(adj.dL, L[0])) * hom.coef - hom.coef_l);
         const MediumInfo &M = S.media[S.hom_medium];
         if (M.albedo_param >= 0 && G->g[M.albedo_param]) {

@@ -223,3 +223,25 @@ def test_one_pass_adjoint_is_the_transpose_of_forward_mode(cuda, max_depth):
         # terms of both signs: float32 rounding of their absolute sum
         size = float((g.double() * fwd.abs()).sum())
         assert size > 0 and abs(lhs - rhs) <= 1e-5 * size, (k, lhs, rhs, size)
+
+
+def test_one_pass_adjoint_of_paths_without_radiance(cuda):
+    # A medium of extinction 0 behind an open null rectangle: its paths leave
+    # towards infinity with throughput 0, and gather nothing. Their terms are
+    # none, not 0 x infinity; pixels beside the rectangle see the environment.
+    announce("homogeneous adjoint, extinction 0, unbounded medium")
+    medium = {"type": "homogeneous", "sigma_t": {"type": "spectrum", "value": 0.0},
+              "albedo": {"type": "rgb", "value": 0.7}, "scale": 2.0}
+    d = homogeneous_box_scene(w=16, h=12, spp=4)
+    d["box"] = {"type": "rectangle", "bsdf": {"type": "null"}, "to_world": T.translate([0.5, 0.5, 1.0]).scale(0.4),
+                "interior": {"type": "twostatemedium", "old": medium, "new": medium, "incoming": medium}}
+    sc = rcv.load_dict(d)
+    p = rcv.traverse(sc)
+    key = [k for k in p.keys() if "sigma_t" in k][0]
+    p[key] = p[key].detach().clone().requires_grad_(True)
+    p.update()
+    integ = rcv.load_dict({"type": "twostateprbvolpath", "max_depth": 6, "rr_depth": 6})
+    img = integ.render(sc, 0, 3, 4)
+    assert float(img.max()) == 1.0 and float(img.min()) == 0.0
+    g = integ.adjoint(sc, p, torch.ones(12, 16, 3, device="cuda"), 0, 3, 4)[key]
+    assert float(g) == 0.0
