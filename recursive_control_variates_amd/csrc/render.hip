@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(kWave
 // out, so no wave waits at the end of the launch for a few long pixels. The
 // result per sample is that of adjoint_kernel; only the order of the gradient
 // scatter-adds differs.
-template <int F, int W>
+template <int F, int W, bool ONCE = false>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(W))) void
 adjoint_persistent_kernel(SceneView S, IntegArgs I, int sensor, uint32_t seed, int spp, int chunk_log2,
                           const float *__restrict__ grad_img, GradTargets G, unsigned *queue, unsigned total_units) {
@@ -219,7 +219,7 @@ adjoint_persistent_kernel(SceneView S, IntegArgs I, int sensor, uint32_t seed, i
   const SensorInfo &sen = S.sensors[sensor];
   const int film_w = sen.film_w;
   LocalCounters cnt{S.counters};
-  VolPath<1, true, F> t;
+  VolPath<1, true, F, false, ONCE> t;
   t.L[0] = v3(0.f);
   t.init_hom();
   log_begin(G, stack);
@@ -727,10 +727,10 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
     GradTargets GL = G;
     // only constants of the homogeneous medium to differentiate
     const int hom = s->view.hom_medium;
-    GL.hom_once = hom >= 0;
+    bool hom_once = hom >= 0;
     for (int i = 0; i < n_params; ++i)
       if (hom < 0 || (param_ids[i] != s->media[hom].sigma_param && param_ids[i] != s->media[hom].albedo_param))
-        GL.hom_once = false;
+        hom_once = false;
     LogLaunch log;
     if (!taped) open_log(s, G, stream, log, GL, n_pix * spp);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, stream, tmp.queue);
@@ -748,11 +748,14 @@ int launch_adjoint(const Scene *s, const rcv_integrator_desc *d, int sensor, uin
           hipLaunchKernelGGL(kern, dim3(pgrid), dim3(block), stack_bytes(block), stream, s->view, I, sensor, seed, spp,
                              ucl2, grad_img, GL, tmp.queue, units);
         };
+        if constexpr ((F & kFeatHomog) != 0) {
+          if (hom_once) return go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint, true>);
+        }
         // three waves per SIMD with the log or without scatter-adds, four
         // with atomics (kWavesPerEuLoggedAdjoint)
         if constexpr (kTapeAdjoint<F>)
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);
-        else if (log.target.g || GL.hom_once)
+        else if (log.target.g)
           go(adjoint_persistent_kernel<F, kWavesPerEuLoggedAdjoint>);
         else
           go(adjoint_persistent_kernel<F, kWavesPerEu<RCV_INTEGRATOR_VOLPATH>>);

@@ -54,8 +54,6 @@ struct GradTargets {
   unsigned log_bin0;
   int log_shift;
   int log_param;
-  // every target is a constant of the homogeneous medium: one pass (HomSum)
-  bool hom_once;
   __host__ __device__ void clear() {
     for (int i = 0; i < kMaxParams; ++i) g[i] = nullptr;
     log_rec = nullptr;
@@ -65,7 +63,6 @@ struct GradTargets {
     log_bin0 = 0;
     log_shift = 0;
     log_param = -1;
-    hom_once = false;
   }
 };
 
@@ -804,18 +801,20 @@ constexpr bool kTapeAdjoint = (F & kFeatSupergrid) && !(F & kFeatAlbedoGrid);
 // every event adds to per-lane sums, which a kernel reduces over its
 // wavefront and adds to the gradient once, at its end (flush_homogeneous).
 //
-// When these are the only targets (GradTargets::hom_once) the primal pass
-// gathers all that its path needs: each event's term is a coefficient times
+// When these are the only targets (VolPath's ONCE) the primal pass gathers all
+// that its path needs: each event's term is a coefficient times
 // the radiance still to come, L less what was gathered before it, so the
 // sums of the coefficients and of coefficient x gathered radiance give the
 // path's terms once L is known, and no path is traced a second time (Cornell
-// box with a homogeneous sphere, 128^2, 16 samples: adjoint 916 -> 590 us).
+// box with a homogeneous sphere, 128^2, 16 samples: adjoint 916 -> 535 us).
 struct HomSum {
   float s;  // d/d(sigma_t value)
   V3 a;     // d/d(albedo)
-  // of the path under way (hom_once): sum of coefficients, of coefficient x
-  // dLoss/dL . gathered (the terms are differences of the two: in 64 bits);
-  // real collisions, radiance gathered at them
+};
+struct HomOnceSum : HomSum {
+  // of the path under way: sum of coefficients, of coefficient x dLoss/dL .
+  // gathered (the terms are differences of the two: in 64 bits); real
+  // collisions, radiance gathered at them
   double coef, coef_l;
   float n;
   V3 l;
@@ -855,8 +854,12 @@ __device__ inline void flush_homogeneous(const SceneView &S, const GradTargets &
 // replays the same random numbers and scatters as it goes. FWD (with ADJ) is
 // forward mode: the replay pass gathers the tangents (in G) where the
 // adjoint scatters and adds d(radiance)/d(theta) . tangent to adj.dI, the
-// transpose of the adjoint on the same samples.
-template <int NS, bool ADJ, int F, bool FWD = false>
+// transpose of the adjoint on the same samples. ONCE: the adjoint of nothing
+// but the homogeneous medium's constants, in one pass (HomOnceSum); a kernel of
+// its own, since its sums beside the replay's state make the others spill
+// (homogeneous medium beside a heterogeneous one in a Cornell box, 128^2, 16
+// samples: adjoint 4990 us in one kernel, 4260 apart).
+template <int NS, bool ADJ, int F, bool FWD = false, bool ONCE = false>
 struct VolPath {
   static_assert(!FWD || ADJ, "forward mode replays paths as the adjoint does");
   static constexpr bool kTape = ADJ && !FWD && kTapeAdjoint<F>;
@@ -871,13 +874,14 @@ struct VolPath {
   AdjState adj;
   std::conditional_t<kTape, PathTape, NoTape> tape;
   static constexpr bool kNeeInline = ADJ && !FWD && !kTape;
-  static constexpr bool kHomOnce = kNeeInline && (F & kFeatHomog) != 0;
+  static constexpr bool kHomAdj = kNeeInline && (F & kFeatHomog) != 0;
+  static_assert(!ONCE || kHomAdj, "one pass for the homogeneous medium's adjoint only");
   std::conditional_t<kNeeInline, NeeWeights, NoNeeWeights> neew;
   // Renders of scenes without surfaces defer the ratio tracking of NEE
   // shadow rays to the following bounce() calls (nee_start).
   static constexpr bool kDeferNee = !ADJ && !(F & kFeatSurfaces);
   bool in_nee;
-  std::conditional_t<ADJ && (F & kFeatHomog) != 0, HomSum, NoHomSum> hom;
+  std::conditional_t<ONCE, HomOnceSum, std::conditional_t<ADJ && (F & kFeatHomog) != 0, HomSum, NoHomSum>> hom;
 
   // Zeroes the homogeneous-medium sums (once per lane, before its samples).
   __device__ void init_hom() {
@@ -907,7 +911,7 @@ struct VolPath {
     last_p = v3(0.f);
     last_pdf = 1.0f;
     medium = -1;
-    replay = ADJ && is_replay;
+    replay = ADJ && !ONCE && is_replay;
     nee_grad = false;
     in_nee = false;
     (void)rng.next_1d();  // colour channel for free-flight sampling (:171-173)
@@ -922,7 +926,7 @@ struct VolPath {
   __device__ void begin_adjoint(const Pcg32 &r, const Ray &camera, LocalCounters &cnt, bool is_replay, V3 dL,
                                 V3 Lp) {
     begin(r, camera, cnt, is_replay);
-    if constexpr (ADJ && (F & kFeatHomog) != 0) {
+    if constexpr (ONCE) {
       hom.coef = hom.coef_l = 0.0;
       hom.n = 0.0f;
       hom.l = v3(0.f);
@@ -941,21 +945,19 @@ struct VolPath {
   // done (its taped collisions scattered), false when it needs its replay
   // pass (an untaped kernel, or a tape overflow).
   __device__ bool end_adjoint(const SceneView &S, LocalCounters &cnt, const GradTargets *G) {
-    if constexpr (kHomOnce) {
-      if (G->hom_once) {
-        // (a path without radiance may hold infinite coefficients: a medium
-        // of extinction 0 left towards infinity)
-        if (!any_nonzero(L[0])) return true;
-        hom.s += float(double(dot(adj.dL, L[0])) * hom.coef - hom.coef_l);
-        const MediumInfo &M = S.media[S.hom_medium];
-        if (M.albedo_param >= 0 && G->g[M.albedo_param]) {
-          const float *al = S.params[M.albedo_param].data[RCV_STATE_NEW];
-          const V3 dl = adj.dL * (L[0] * hom.n - hom.l);
-          hom.a += v3(al[0] != 0.f ? dl.x / al[0] : 0.f, al[1] != 0.f ? dl.y / al[1] : 0.f,
-                      al[2] != 0.f ? dl.z / al[2] : 0.f);
-        }
-        return true;
+    if constexpr (ONCE) {
+      // (a path without radiance may hold infinite coefficients: a medium of
+      // extinction 0 left towards infinity)
+      if (!any_nonzero(L[0])) return true;
+      hom.s += float(double(dot(adj.dL, L[0])) * hom.coef - hom.coef_l);
+      const MediumInfo &M = S.media[S.hom_medium];
+      if (M.albedo_param >= 0 && G->g[M.albedo_param]) {
+        const float *al = S.params[M.albedo_param].data[RCV_STATE_NEW];
+        const V3 dl = adj.dL * (L[0] * hom.n - hom.l);
+        hom.a += v3(al[0] != 0.f ? dl.x / al[0] : 0.f, al[1] != 0.f ? dl.y / al[1] : 0.f,
+                    al[2] != 0.f ? dl.z / al[2] : 0.f);
       }
+      return true;
     }
     if constexpr (kTape) {
       if (replay || !any_nonzero(L[0])) return true;
@@ -1004,14 +1006,10 @@ struct VolPath {
       // contribution
       if (nee_grad && any_nonzero(c[0])) adj.dI += c[0] * tsum;
     }
-    if constexpr (kHomOnce) {
+    if constexpr (ONCE) {
       // hom_seg: the shadow ray's d(log T)/d(value)
-      if (G->hom_once) {
-        hom.s += dot(adj.dL, c[0]) * hom_seg;
-        return;
-      }
-    }
-    if constexpr (kNeeInline) {
+      hom.s += dot(adj.dL, c[0]) * hom_seg;
+    } else if constexpr (kNeeInline) {
       if (!replay) {
         if (neew.k < stack.nslots - 1) stack.slot(neew.k) = __float_as_int(dot(adj.dL, c[0]));
       } else if (!have_cs) {
@@ -1280,8 +1278,7 @@ struct VolPath {
       }
     }
     if constexpr (ADJ && (F & kFeatHomog) != 0) {
-      const bool once = kHomOnce && G->hom_once;
-      if ((replay || once) && in_hom && (escaped || active_medium)) {
+      if ((replay || ONCE) && in_hom && (escaped || active_medium)) {
         // d log(weight)/d(value) (sigma_t = scale value) of this segment's
         // weight times the radiance it multiplies: null collision -scale /
         // sigma_n, real collision +scale / sigma_t; without null scattering
@@ -1305,7 +1302,7 @@ struct VolPath {
               adj.dI += adj.Lrem * v3(mev.alb.x != 0.f ? ta[0] / mev.alb.x : 0.f,
                                       mev.alb.y != 0.f ? ta[1] / mev.alb.y : 0.f,
                                       mev.alb.z != 0.f ? ta[2] / mev.alb.z : 0.f);
-        } else if (once) {
+        } else if constexpr (ONCE) {
           hom.coef += double(coef);
           hom.coef_l += double(coef) * double(dot(adj.dL, L[0]));
           if (act_scatter) {
@@ -1446,16 +1443,13 @@ struct VolPath {
         if constexpr (ADJ) {
           // one instantiation for both passes, so that they compute the same
           // transmittance from the same random numbers
-          float *hacc = nullptr;
-          if constexpr (kNeeInline && (F & kFeatHomog) != 0) hacc = have_cs ? &hom.s : nullptr;
-          if constexpr (kHomOnce) {
-            if (G->hom_once) {
-              cs_in = 1.0f;
-              hacc = &hom_seg;
-            }
-          }
+          if (ONCE) cs_in = 1.0f;
           nee_twostates<NS, true, F>(S, ref_p, si.n, active_e_surface, medium, rng, em, ds, stack, cnt, cs_in, G,
-                                     kTape && nee_grad ? &rec : nullptr, hacc, FWD && nee_grad ? &tsum : nullptr);
+                                     kTape && nee_grad ? &rec : nullptr, kHomAdj ? &hom_seg : nullptr,
+                                     FWD && nee_grad ? &tsum : nullptr);
+          if constexpr (kHomAdj && !ONCE) {
+            if (have_cs) hom.s += hom_seg;
+          }
         } else {
           nee_twostates<NS, false, F>(S, ref_p, si.n, active_e_surface, medium, rng, em, ds, stack, cnt, 0.f, G);
         }
