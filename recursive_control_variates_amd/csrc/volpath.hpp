@@ -576,7 +576,7 @@ __device__ inline bool shadow_step(const SceneView &S, Shadow<NS> &sh, SurfInt &
   if (!(remaining > 0.0f)) return false;
   if (sh.needs_int) {
     Hit h;
-    trace<false>(S, sh.ray, h, stack);
+    trace<false, (F & kFeatHomog) != 0>(S, sh.ray, h, stack);
     cnt.add(kCntTraversals, 1);
     si = make_si(S, sh.ray, h);
     sh.needs_int = false;
@@ -1179,7 +1179,7 @@ struct VolPath {
       if (in_hom && mev.valid) ray.maxt = mev.t;
       if (needs_int) {
         Hit h;
-        trace<false>(S, ray, h, stack);
+        trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
         cnt.add(kCntTraversals, 1);
         si = make_si(S, ray, h);
       }
@@ -1374,7 +1374,7 @@ struct VolPath {
     active_surface = active_surface || escaped;
     if (active_surface && needs_int) {
       Hit h;
-      trace<false>(S, ray, h, stack);
+      trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
       cnt.add(kCntTraversals, 1);
       si = make_si(S, ray, h);
     }

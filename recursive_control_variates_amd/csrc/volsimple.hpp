@@ -133,7 +133,7 @@ __device__ inline V3 simple_sample_emitter(const SceneView &S, int medium, V3 p,
   r.d = ds.d;
   r.maxt = kInf;
   Hit h;
-  trace<false>(S, r, h, stack);
+  trace<false, (F & kFeatHomog) != 0>(S, r, h, stack);
   cnt.add(kCntTraversals, 1);
   const SurfInt si = make_si(S, r, h);
   if (!si.valid) return v3(0.f);
@@ -213,7 +213,7 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
     cnt.add(kCntPaths, 1);
     (void)rng.next_1d();  // colour channel (:86)
     Hit h;
-    trace<false>(S, ray, h, stack);
+    trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
     cnt.add(kCntTraversals, 1);
     const SurfInt s0 = make_si(S, ray, h);
     escaped = !s0.valid;
@@ -221,7 +221,7 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
     si = s0;
     if (active) {
       ray = spawn_ray(s0, ray.d);
-      trace<false>(S, ray, h, stack);
+      trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
       cnt.add(kCntTraversals, 1);
       si = make_si(S, ray, h);
       active = si.valid;
@@ -376,7 +376,7 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
     if (did_scatter || did_escape) {
       ray.maxt = kInf;
       Hit h;
-      trace<false>(S, ray, h, stack);
+      trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
       cnt.add(kCntTraversals, 1);
       si = make_si(S, ray, h);
       ray.maxt = si.valid ? si.t : kInf;
@@ -403,7 +403,7 @@ __device__ V3 simple_sample(const SceneView &S, const IntegArgs &I, int medium, 
   if (escaped) {
     ray.maxt = kInf;
     Hit h;
-    trace<false>(S, ray, h, stack);
+    trace<false, (F & kFeatHomog) != 0>(S, ray, h, stack);
     cnt.add(kCntTraversals, 1);
     const SurfInt se = make_si(S, ray, h);
     const int em = si_emitter(S, se);
@@ -499,7 +499,7 @@ __device__ V3 simple_recursive_li(const SceneView &S, const IntegArgs &I, int me
   rec.d = square_to_uniform_sphere(a, b);
   rec.maxt = kInf;
   Hit h;
-  trace<false>(S, rec, h, stack);
+  trace<false, (F & kFeatHomog) != 0>(S, rec, h, stack);
   cnt.add(kCntTraversals, 1);
   SimpleStart st;
   st.from_camera = false;
