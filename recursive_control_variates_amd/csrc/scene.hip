@@ -199,7 +199,8 @@ __global__ __launch_bounds__(1024) void max_reduce_kernel(const float *__restric
 // The planar primitives of a scene of few triangles: pairs of consecutive
 // triangles of a shape that form a parallelogram, and the other triangles. In
 // double, from the triangles' float corners. Empty when there are more than
-// kMaxFlat of them, or one is degenerate.
+// kMaxFlat of them, or one is more slender than flat_trace's error bound allows
+// (kMaxSlender) or degenerate.
 static std::vector<FlatPrim> flat_prims(const std::vector<float> &tri_v, const std::vector<int32_t> &tri_shape,
                                         const std::vector<int32_t> &slot_of) {
   std::vector<FlatPrim> out;
@@ -233,7 +234,9 @@ static std::vector<FlatPrim> flat_prims(const std::vector<float> &tri_v, const s
     }
     const P m = cross3(a, b);
     const double len = std::sqrt(dot3(m, m));
-    if (!(len > 1e-10) || int(out.size()) == kMaxFlat) return {};
+    const P c = sub(b, a);
+    const double longest = std::max(dot3(a, a), std::max(dot3(b, b), dot3(c, c)));
+    if (!(len > 1e-10) || longest > kMaxSlender * len || int(out.size()) == kMaxFlat) return {};
     const P nn = {m[0] / len, m[1] / len, m[2] / len};
     // dual basis: A . a = 1, A . b = 0, A . n = 0
     P A = cross3(b, nn), B = cross3(nn, a);

@@ -225,7 +225,8 @@ __device__ inline LdsStack lds_of(const SceneView &S, int *lds) {
 // The result is the BVH's bit for bit: plane and edge tests in plain
 // arithmetic only decide which primitive is hit, and only when they decide it
 // beyond their own rounding error (`eps`, a bound of the position error) and
-// beyond that of the exact triangle test; then that test gives the hit. -1
+// beyond that of the exact triangle test, both of which grow as a triangle gets
+// slender (kMaxSlender); then that test gives the hit. -1
 // for a ray nearer to an edge, a diagonal, a plane or a tie than that: the
 // caller takes the BVH.
 template <bool ANY_HIT>

@@ -93,3 +93,55 @@ def test_flat_trace_of_axis_parallel_and_edge_rays(cuda, name):
         imgs.append(rcv.load_dict({"type": kind, "max_depth": 3}).render(sc, 0, 4, 8).cpu().numpy())
     off = (np.abs(imgs[0] - imgs[1]) > 1e-5 * np.abs(imgs[1]) + 1e-6).any(axis=-1).sum()
     assert off <= 1, off
+
+
+# Triangles whose longest edge squared is 650 to 1400 times twice their area,
+# with a ray that passes an edge by a few of flat_trace's error bounds: corners,
+# origin and aim. The exact test's rounding decides such rays, which differs
+# from that of the plane arithmetic.
+SLENDER = [
+    ([(-0.574098408, -0.84156394, 0.271853179),
+      (-0.662747085, -0.919269085, -0.163141653),
+      (-0.662446916, -0.919084191, -0.163264483)],
+     (1.30990362, -2.12933588, -0.582932115), (-0.662626272, -0.919196959, -0.163237821)),
+    ([(0.888710678, -0.667799354, -0.913880408),
+      (0.571613371, -0.393958598, -0.971578956),
+      (0.571358919, -0.39413932, -0.971578598)],
+     (0.825455368, -1.57785404, -2.64932489), (0.571582298, -0.39398066, -0.971578913)),
+    ([(-0.0412372611, 0.230409771, -0.376535982),
+      (-0.655070186, -0.453622699, -0.436333328),
+      (-0.653996944, -0.454530478, -0.436249822)],
+     (-2.47753286, 0.158143461, -2.20428133), (-0.654465049, -0.454185023, -0.436286749)),
+    ([(-0.819045722, -0.0108747967, -0.633749902),
+      (-1.36246324, -0.496002436, -1.31658602),
+      (-1.36244345, -0.495248348, -1.31685078)],
+     (0.355672807, -1.84802747, -1.72207677), (-1.3624468, -0.495381475, -1.31680382)),
+    ([(-0.950862288, -0.0256499425, 0.176232278),
+      (-0.389036149, -0.241063565, 0.56866312),
+      (-0.389438152, -0.240668342, 0.567294121)],
+     (-0.732924759, 1.57457078, 1.70631206), (-0.389320577, -0.240788209, 0.567713812)),
+    ([(-0.831167579, 0.328666508, 0.910116732),
+      (-1.35111499, 0.174996153, 0.382492304),
+      (-1.3512727, 0.174067885, 0.382832378)],
+     (0.381067455, 1.45943701, -0.869288862), (-1.35120776, 0.174449847, 0.382692501)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(SLENDER)))
+def test_flat_trace_of_slender_triangles(cuda, case):
+    # a film 3e-5 wide around the aim, most of it within the rounding of the edge
+    announce(f"flat trace of a slender triangle ({case})")
+    corners, origin, aim = SLENDER[case]
+    dist = np.linalg.norm(np.subtract(origin, aim))
+    imgs = []
+    for hidden in (False, True):
+        d = {"type": "scene", "tri": _tri(corners, 0.4),
+             "env": {"type": "constant", "radiance": {"type": "rgb", "value": 1.0}},
+             "ball": {"type": "sphere", "center": [0, -1.6, 0], "radius": 0.3,
+                      "bsdf": {"type": "diffuse", "reflectance": {"type": "rgb", "value": 0.5}}},
+             "sensor": cam(origin, aim, fov=float(np.degrees(3e-5 / dist)), w=32, h=32, spp=16)}
+        if hidden:
+            d["hidden"] = _hidden((0, -1.6, 0))
+        imgs.append(rcv.load_dict({"type": "prb", "max_depth": 2}).render(rcv.load_dict(d), 0, 9, 16).cpu().numpy())
+    off = (np.abs(imgs[0] - imgs[1]) > 1e-5 * np.abs(imgs[1]) + 1e-6).any(axis=-1).sum()
+    assert off <= 1, off
