@@ -161,8 +161,7 @@ __device__ inline void record_corners(const float4 &e, const LogTarget &T, const
   }
 }
 
-// Largest magnitude of the records of each bin (the bits of a non-negative
-// float compare as an integer; NaN counts as inf), for a log whose bins hold
+// Sum of the magnitudes of each bin's records, for a log whose bins hold
 // several tiles: one pass over the records instead of one per tile.
 constexpr int kBoundBlock = int(kLogChunk);
 constexpr int kBoundUnroll = 4;
@@ -170,9 +169,9 @@ constexpr int kBoundBlocks = 1024;
 __global__ __launch_bounds__(kBoundBlock) void log_bound_kernel(const float4 *__restrict__ rec,
                                                                 const unsigned *__restrict__ ctl,
                                                                 const unsigned *__restrict__ meta, unsigned nchunks,
-                                                                unsigned *bound) {
-  __shared__ unsigned top[kLogBins];
-  if (threadIdx.x < unsigned(kLogBins)) top[threadIdx.x] = 0u;
+                                                                float *bound) {
+  __shared__ float sum[kLogBins];
+  if (threadIdx.x < unsigned(kLogBins)) sum[threadIdx.x] = 0.0f;
   __syncthreads();
   const unsigned drawn = min(*ctl, nchunks);
   constexpr unsigned kFillMask = (1u << kLogFillBits) - 1u;
@@ -187,35 +186,36 @@ __global__ __launch_bounds__(kBoundBlock) void log_bound_kernel(const float4 *__
     }
 #pragma unroll
     for (int u = 0; u < kBoundUnroll; ++u) {
-      const float a = fabsf(w[u]);
-      float t = a == a ? a : INFINITY;
-      for (int off = 32; off > 0; off >>= 1) t = fmaxf(t, __shfl_xor(t, off, 64));
-      if ((threadIdx.x & 63u) == 0 && t > 0.0f)
-        atomicMax(&top[(m[u] >> kLogFillBits) % unsigned(kLogBins)], __float_as_uint(t));
+      float t = fabsf(w[u]);
+      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      if ((threadIdx.x & 63u) == 0 && t != 0.0f) atomicAdd(&sum[(m[u] >> kLogFillBits) % unsigned(kLogBins)], t);
     }
   }
   __syncthreads();
-  if (threadIdx.x < unsigned(kLogBins) && top[threadIdx.x] != 0u) atomicMax(bound + threadIdx.x, top[threadIdx.x]);
+  if (threadIdx.x < unsigned(kLogBins) && sum[threadIdx.x] != 0.0f) atomicAdd(bound + threadIdx.x, sum[threadIdx.x]);
 }
 
 // Adds the scatter log of a launch to its gradients, tile by tile (block y:
 // a tile of one of n targets; `one` for n = 1). The tile is summed in LDS in
 // 64-bit fixed point: integer LDS atomics run ~5x faster than float ones
-// here. A first pass over the share's values finds its record count N and
-// largest magnitude M; terms are scaled by 2^s with M N 2^s <= 2^62, so no
-// partial sum overflows and each term is kept to ~2^-44 of M (float atomics
-// keep 2^-24 of the running sum). A share holding a non-finite value is
-// summed with float atomics as it stands. WIDE: a log whose bins hold several
-// tiles; M is then its bins' (`bound`), N the share's count from its chunks.
+// here. A first pass over the share finds the sum M of its records'
+// magnitudes; terms are scaled by 2^s with M 2^s <= 2^62 (float rounding adds
+// less than 2^-9 to that), so no partial sum overflows and each term is kept to
+// 2^-62 of M: as exactly as its float value for voxels down to 2^-38 of M,
+// where float atomics keep 2^-24 of the running sum. (The largest magnitude
+// times the count in place of M, up to 2^23 times as much, cost as many bits.)
+// A share holding a non-finite value is summed with float atomics as it
+// stands. WIDE: a log whose bins hold several tiles; M is then its bins' sum
+// (`bound`), over all shares.
 template <bool WIDE>
 __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *__restrict__ rec,
                                                                   const unsigned *__restrict__ ctl,
                                                                   const unsigned *__restrict__ meta, unsigned nchunks,
                                                                   LogTarget one, const LogTarget *__restrict__ many,
                                                                   int n, int tile_voxels,
-                                                                  const unsigned *__restrict__ bound) {
+                                                                  const float *__restrict__ bound) {
   extern __shared__ long long acc[];  // tile words (floats in the first half for a non-finite share)
-  __shared__ float wave_max[kReduceBlock / 64];
+  __shared__ float wave_sum[kReduceBlock / 64];
   __shared__ unsigned wave_count[kReduceBlock / 64];
   __shared__ unsigned wave_chunks[kReduceBlock / 64];
   __shared__ unsigned picked[kReduceBlock];
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
   float m = 0.0f;
   unsigned total = 0, chunks = 0;
   if constexpr (WIDE) {
-    // the bins' magnitudes are known; the record count from the chunks'
+    // the bins' sums are known; how full the chunks are
     for (unsigned c = blockIdx.x + threadIdx.x * gridDim.x; c < drawn; c += gridDim.x * unsigned(kReduceBlock)) {
       const unsigned w = meta[c];
       const unsigned fill = w & ((1u << kLogFillBits) - 1u);
@@ -244,40 +244,40 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
         ++chunks;
       }
     }
-    m = __uint_as_float(bound[bins.bin]);
-    if (bins.after) m = fmaxf(m, __uint_as_float(bound[kLogMaxTiles + bins.bin]));
-    if (bins.before) m = fmaxf(m, __uint_as_float(bound[kLogMaxTiles + bins.bin - 1]));
   } else {
-    log_block_records<false>(rec, meta, drawn, T, bins, picked, &n_picked, [&](const float4 &e) {
-      const float a = fabsf(e.w);
-      m = (a <= m) ? m : (a == a ? a : INFINITY);  // NaN and inf both give inf
-      ++total;
-    });
+    log_block_records<false>(rec, meta, drawn, T, bins, picked, &n_picked, [&](const float4 &e) { m += fabsf(e.w); });
   }
   for (int off = 32; off > 0; off >>= 1) {
-    m = fmaxf(m, __shfl_xor(m, off, 64));
-    total += __shfl_xor(total, off, 64);
-    chunks += __shfl_xor(chunks, off, 64);
+    m += __shfl_xor(m, off, 64);
+    if constexpr (WIDE) {
+      total += __shfl_xor(total, off, 64);
+      chunks += __shfl_xor(chunks, off, 64);
+    }
   }
   if ((threadIdx.x & 63u) == 0) {
-    wave_max[threadIdx.x >> 6] = m;
+    wave_sum[threadIdx.x >> 6] = m;
     wave_count[threadIdx.x >> 6] = total;
     wave_chunks[threadIdx.x >> 6] = chunks;
   }
   __syncthreads();
-  m = 0.0f;
-  total = chunks = 0;
-  for (int w = 0; w < kReduceBlock / 64; ++w) {
-    m = fmaxf(m, wave_max[w]);
-    total += wave_count[w];
-    chunks += wave_chunks[w];
+  if constexpr (WIDE) {
+    total = chunks = 0;
+    for (int w = 0; w < kReduceBlock / 64; ++w) {
+      total += wave_count[w];
+      chunks += wave_chunks[w];
+    }
+    if (total == 0) return;
+    m = bound[bins.bin] + (bins.after ? bound[kLogMaxTiles + bins.bin] : 0.0f) +
+        (bins.before ? bound[kLogMaxTiles + bins.bin - 1] : 0.0f);
+  } else {
+    m = 0.0f;
+    for (int w = 0; w < kReduceBlock / 64; ++w) m += wave_sum[w];
   }
-  if (total == 0 || m == 0.0f) return;
+  if (m == 0.0f) return;
   if (isfinite(m)) {
-    int em = 0, en = 0;
-    (void)frexpf(m, &em);               // m < 2^em
-    (void)frexpf(float(total), &en);    // total <= 2^en
-    const int sc = 62 - em - en;
+    int em = 0;
+    (void)frexpf(m, &em);  // m < 2^em
+    const int sc = 62 - em;
     for (int v = threadIdx.x; v < tile_voxels; v += blockDim.x) acc[v] = 0;
     __syncthreads();
     // (scaled before the weights: the same products times 2^sc)
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kReduceBlock) void log_reduce_kernel(const float4 *
 
 __global__ void zero_ctl_kernel(unsigned *p) { p[threadIdx.x] = 0u; }
 
-// Chunks drawn, then the bins' magnitudes (log_bound_kernel).
+// Chunks drawn, then the bins' sums (log_bound_kernel).
 constexpr int kCtlWords = 1 + kLogBins;
 
 int allocate(LogBuf &out) {
@@ -455,14 +455,14 @@ void reduce_log(const LogLaunch &log, const GradTargets &GL, hipStream_t stream)
   const size_t lds = size_t(tile) * sizeof(long long);
   const LogTarget *const none = nullptr;
   if ((1 << log.target.shift) > tile) {
-    unsigned *const bound = L.ctl + 1;
+    float *const bound = reinterpret_cast<float *>(L.ctl + 1);
     hipLaunchKernelGGL(log_bound_kernel, dim3(kBoundBlocks), dim3(kBoundBlock), 0, stream, L.rec, L.ctl, L.meta,
                        GL.log_chunks, bound);
     hipLaunchKernelGGL(log_reduce_kernel<true>, grid, dim3(kReduceBlock), lds, stream, L.rec, L.ctl, L.meta,
                        GL.log_chunks, log.target, none, 1, tile, bound);
   } else {
     hipLaunchKernelGGL(log_reduce_kernel<false>, grid, dim3(kReduceBlock), lds, stream, L.rec, L.ctl, L.meta,
-                       GL.log_chunks, log.target, none, 1, tile, static_cast<const unsigned *>(nullptr));
+                       GL.log_chunks, log.target, none, 1, tile, static_cast<const float *>(nullptr));
   }
 }
 
@@ -477,7 +477,7 @@ void reduce_log_batch(const LogBuf &buf, const LogTarget &first, const LogTarget
   const int splits = std::min(kLogSplits, std::max(5, odd_splits(4096 / tiles)));
   hipLaunchKernelGGL(log_reduce_kernel<false>, dim3(splits, tiles), dim3(kReduceBlock), size_t(tile) * sizeof(long long),
                      stream, buf.rec, buf.ctl, buf.meta, log_pool_chunks(), first, targets, n, tile,
-                     static_cast<const unsigned *>(nullptr));
+                     static_cast<const float *>(nullptr));
 }
 
 bool take_log_pool(LogBuf &buf) {

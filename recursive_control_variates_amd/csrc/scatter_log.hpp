@@ -13,7 +13,7 @@ constexpr unsigned kLogPool = 786432;
 
 struct LogBuf {
   float4 *rec = nullptr;
-  unsigned *ctl = nullptr;   // chunks drawn, bins' magnitudes
+  unsigned *ctl = nullptr;   // chunks drawn, bins' sums of magnitudes
   unsigned *meta = nullptr;  // kLogPool chunk bins and record counts
 };
 

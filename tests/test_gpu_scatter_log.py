@@ -55,3 +55,32 @@ def test_media_over_one_grid(cuda, same_place):
     scale = np.abs(out[1]).max()
     assert scale > 0
     assert np.allclose(out[0], out[1], rtol=1e-4, atol=1e-4 * scale), np.abs(out[0] - out[1]).max() / scale
+
+
+# (the last one's bins hold several reduction tiles)
+@pytest.mark.parametrize("kind,n,w,h,spp", [("prbvolpath", 20, 48, 32, 16), ("volpathsimple", 20, 48, 32, 16),
+                                            ("prbvolpath", 72, 256, 256, 8)])
+def test_small_sums_beside_large_records(cuda, kind, n, w, h, spp):
+    # One pixel of the image gradient is 2^38 times the others. Voxels its paths
+    # do not reach get the other pixels' terms alone, of 10 or so times 2^-38
+    # each, in the same bins as its records, whose magnitudes sum to about 2^11:
+    # kept to 2^-62 of that, a voxel's ~100 terms are off by 2^-48 together,
+    # 2^-13 of their sum. With the largest record (2^6) times the count (2^13 in
+    # a share) in the sum's place it would be 2^-5.
+    announce(f"scatter log, small sums beside large records ({kind}, {n}^3)")
+    rng = np.random.default_rng(79)
+    grid = (0.2 + rng.uniform(0, 0.8, (n, n, n, 1))).astype(np.float32)
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=0.8, scale=5.0, w=w, h=h, spp=spp))
+    p = rcv.traverse(sc)
+    p[KEY] = p[KEY].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    integ = rcv.load_dict({"type": kind, "max_depth": 3, "rr_depth": 8})
+    one = torch.zeros(h, w, 3, device="cuda")
+    one[h // 2, w // 2] = 1.0
+    rest = torch.full_like(one, 2.0 ** -38) * (one == 0)
+    g1, g2, g = (integ.adjoint(sc, p, x, 0, 83, spp)[KEY].double().cpu().numpy() for x in (one, rest, one + rest))
+    apart = (g1 == 0) & (g2 != 0)
+    assert apart.sum() > 0.1 * n ** 3 and np.abs(g1).max() > 1e8 * np.abs(g2).max()
+    off = np.abs(g - g2)[apart]
+    assert off.max() <= 2e-3 * np.abs(g2[apart]).mean(), off.max() / np.abs(g2[apart]).mean()
