@@ -397,6 +397,13 @@ constexpr int kLogNext = kLogBins - 1, kLogEnd = 2 * kLogBins - 1;
 __device__ inline int *wave_log_word(const LdsStack &L, int lane) {
   return L.base + (kLdsWordsPerThread - 1) * L.stride - int(threadIdx.x & 63u) + lane;
 }
+// (one lane writes what others read: atomic, so that no lane keeps a value)
+__device__ inline int log_load(const LdsStack &L, int lane) {
+  return __hip_atomic_load(wave_log_word(L, lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ inline void log_store(const LdsStack &L, int lane, int v) {
+  __hip_atomic_store(wave_log_word(L, lane), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 
 __device__ inline unsigned log_meta_of(const GradTargets &G, int bin, unsigned fill) {
   return ((G.log_bin0 + unsigned(bin)) << kLogFillBits) | min(fill, kLogChunk);
@@ -405,7 +412,7 @@ __device__ inline unsigned log_meta_of(const GradTargets &G, int bin, unsigned f
 // Before the wavefront's first scatter: no chunk in any bin, none drawn.
 __device__ inline void log_begin(const GradTargets &G, const LdsStack &L) {
   const int lane = int(threadIdx.x & 63u);
-  if (G.log_rec) *wave_log_word(L, lane) = lane < kLogNext ? -1 : 0;
+  if (G.log_rec) log_store(L, lane, lane < kLogNext ? -1 : 0);
 }
 
 // With the whole wavefront past its last scatter into G's gradient: the
@@ -413,10 +420,10 @@ __device__ inline void log_begin(const GradTargets &G, const LdsStack &L) {
 __device__ inline void log_close(const GradTargets &G, const LdsStack &L) {
   const int lane = int(threadIdx.x & 63u);
   if (G.log_rec && lane < kLogNext) {
-    const int c = *wave_log_word(L, lane);
-    if (c >= 0) G.log_meta[c] = log_meta_of(G, lane, unsigned(*wave_log_word(L, kLogBins + lane)));
-    *wave_log_word(L, lane) = -1;
-    *wave_log_word(L, kLogBins + lane) = 0;
+    const int c = log_load(L, lane);
+    if (c >= 0) G.log_meta[c] = log_meta_of(G, lane, unsigned(log_load(L, kLogBins + lane)));
+    log_store(L, lane, -1);
+    log_store(L, kLogBins + lane, 0);
   }
 }
 
@@ -424,8 +431,8 @@ __device__ inline void log_close(const GradTargets &G, const LdsStack &L) {
 // use are empty.
 __device__ inline void log_end(const GradTargets &G, const LdsStack &L) {
   if (!G.log_rec) return;
-  const unsigned next = unsigned(*wave_log_word(L, kLogNext));
-  const unsigned end = min(unsigned(*wave_log_word(L, kLogEnd)), G.log_chunks);
+  const unsigned next = unsigned(log_load(L, kLogNext));
+  const unsigned end = min(unsigned(log_load(L, kLogEnd)), G.log_chunks);
   for (unsigned c = next + (threadIdx.x & 63u); c < end; c += 64) G.log_meta[c] = 0;
 }
 
@@ -447,7 +454,7 @@ __device__ inline void scatter_density(const GradTargets *G, const LdsStack &L, 
   const int tile = f.base >> G->log_shift;
   const int bin = ((f.base + f.dx + f.dy + f.dz) >> G->log_shift) == tile ? tile : kLogMaxTiles + tile;
   const float4 rec = make_float4(p.x, p.y, p.z, val);
-  const int chunk = *wave_log_word(L, bin);
+  const int chunk = log_load(L, bin);
   const unsigned r = unsigned(__hip_atomic_fetch_add(wave_log_word(L, kLogBins + bin), 1, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_WAVEFRONT));
   const bool ok = chunk >= 0 && r < kLogChunk;
@@ -463,19 +470,18 @@ __device__ inline void scatter_density(const GradTargets *G, const LdsStack &L, 
   const uint64_t mb = __ballot(!ok && bin == b);
   int c = -1;
   if (lane == leader) {
-    int *const cw = wave_log_word(L, b);
-    int *const fw = wave_log_word(L, kLogBins + b);
-    if (*cw >= 0) G->log_meta[*cw] = log_meta_of(*G, b, unsigned(*fw));
-    unsigned next = unsigned(*wave_log_word(L, kLogNext));
-    const unsigned end = unsigned(*wave_log_word(L, kLogEnd));
+    const int full = log_load(L, b);
+    if (full >= 0) G->log_meta[full] = log_meta_of(*G, b, unsigned(log_load(L, kLogBins + b)));
+    unsigned next = unsigned(log_load(L, kLogNext));
+    const unsigned end = unsigned(log_load(L, kLogEnd));
     if (next >= end && end < G->log_chunks) {  // (no draw once the pool's end is known)
       next = atomicAdd(G->log_ctl, kLogDraw);
-      *wave_log_word(L, kLogEnd) = int(next + kLogDraw);
+      log_store(L, kLogEnd, int(next + kLogDraw));
     }
     if (next < G->log_chunks) c = int(next);
-    *wave_log_word(L, kLogNext) = int(next + 1);
-    *cw = c;
-    *fw = c >= 0 ? int(__popcll(mb)) : 0;
+    log_store(L, kLogNext, int(next + 1));
+    log_store(L, b, c);
+    log_store(L, kLogBins + b, c >= 0 ? int(__popcll(mb)) : 0);
   }
   c = __builtin_amdgcn_readlane(c, leader);
   if (!ok) {
