@@ -84,3 +84,42 @@ def test_small_sums_beside_large_records(cuda, kind, n, w, h, spp):
     assert apart.sum() > 0.1 * n ** 3 and np.abs(g1).max() > 1e8 * np.abs(g2).max()
     off = np.abs(g - g2)[apart]
     assert off.max() <= 2e-3 * np.abs(g2[apart]).mean(), off.max() / np.abs(g2[apart]).mean()
+
+
+# Rows of one voxel, which the one-box tracker leaves to the general kernels;
+# bins of several reduction tiles with an albedo grid and a majorant supergrid.
+@pytest.mark.parametrize("kind,shape,w,h,spp,factor,albedo_grid", [
+    ("prbvolpath", (6, 5, 1), 48, 32, 16, 0, False),
+    ("volpathsimple", (6, 5, 1), 48, 32, 16, 0, True),
+    ("prbvolpath", (72, 66, 70), 256, 256, 8, 0, True),
+    ("prbvolpath", (72, 66, 70), 256, 256, 8, 8, False),
+    ("volpathsimple", (66, 72, 70), 256, 256, 8, 8, True),
+])
+def test_logged_adjoint_equals_static(cuda, kind, shape, w, h, spp, factor, albedo_grid):
+    # The terms are the static launch's, in another order: up to ~10^5 per voxel
+    # of the small grids, sqrt(10^5) 2^-24 = 2e-5 of the largest partial sum,
+    # 1e-4 of the largest gradient with room for partial sums above the result.
+    announce(f"{kind} adjoint, logged vs static, {shape} factor {factor} albedo grid {albedo_grid}")
+    rng = np.random.default_rng(89)
+    grid = (0.2 + rng.uniform(0, 0.8, shape + (1,))).astype(np.float32)
+    albedo, keys = 0.8, [KEY]
+    if albedo_grid:
+        data = rng.uniform(0.3, 0.9, shape + (3,)).astype(np.float32)
+        albedo = {"type": "gridvolume", "data": data, "to_world": T.scale(1.0)}
+        keys.append("box.interior_medium.albedo.data")
+    sc = rcv.load_dict(volume_box_scene(grid, albedo=albedo, scale=5.0, w=w, h=h, spp=spp, majorant_factor=factor))
+    p = rcv.traverse(sc)
+    for k in keys:
+        p[k] = p[k].detach().clone().requires_grad_(True)
+    p.update()
+    p.update()
+    gimg = torch.from_numpy(rng.uniform(0.5, 1.5, (h, w, 3)).astype(np.float32)).cuda()
+    integ = rcv.load_dict({"type": kind, "max_depth": 6, "rr_depth": 4})
+    out = []
+    for spt in (0, 4):
+        integ.samples_per_thread = spt
+        g = integ.adjoint(sc, p, gimg, 0, 97, spp)
+        out.append([g[k].double().cpu().numpy() for k in keys])
+    for a, b in zip(*out):
+        scale = np.abs(b).max()
+        assert scale > 0 and np.allclose(a, b, rtol=1e-4, atol=1e-4 * scale), np.abs(a - b).max() / scale
