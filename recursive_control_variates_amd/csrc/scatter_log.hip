@@ -30,8 +30,8 @@ namespace {
 //
 // A grid of more than kLogMaxTiles tiles has bins of several tiles, and each
 // of them reads its bin's records: 8 times at 128^3, whose step with an albedo
-// grid (192^2 per view, 8 samples) takes 8.8 ms (adjoint 2.8, reduction 2.2,
-// magnitudes 0.09), with atomics 11.7 (adjoint 7.2). Those bins' magnitudes
+// grid (192^2 per view, 8 samples) takes 8.8 ms (adjoint 2.7, reduction 2.3,
+// sums 0.09), with atomics 11.7 (adjoint 7.2). Those bins' sums
 // come from one pass over all records (log_bound_kernel) instead of one per
 // tile: 2.95 -> 2.16 ms of reduction.
 //
@@ -53,8 +53,8 @@ constexpr unsigned kSparseChunks = unsigned(kReduceBlock) / 64u * unsigned(kRedu
 // blocks an eighth of them got all first chunks (two tiles, 262144 samples:
 // 203 us, with 63 blocks 88).
 constexpr int kLogSplits = 63;  // at most
-constexpr int kLogMinSplits = 15;
-constexpr int odd_splits(int n) { return (n - 1) | 1; }
+constexpr int kLogMinSplits = 17;
+constexpr int odd_splits(int n) { return n | 1; }
 static_assert(kLogSplits % 2 == 1 && kLogMinSplits % 2 == 1 && kLogDraw % 2 == 0, "odd against the draw size");
 static_assert(kReduceBlock % int(kLogChunk) == 0 && kLogChunk % 64 == 0,
               "a reduction block covers whole chunks, a wavefront whole rows of one");
@@ -165,7 +165,7 @@ __device__ inline void record_corners(const float4 &e, const LogTarget &T, const
 // several tiles: one pass over the records instead of one per tile.
 constexpr int kBoundBlock = int(kLogChunk);
 constexpr int kBoundUnroll = 4;
-constexpr int kBoundBlocks = 1024;
+constexpr int kBoundBlocks = 2048;
 __global__ __launch_bounds__(kBoundBlock) void log_bound_kernel(const float4 *__restrict__ rec,
                                                                 const unsigned *__restrict__ ctl,
                                                                 const unsigned *__restrict__ meta, unsigned nchunks,
