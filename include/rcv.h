@@ -213,7 +213,7 @@ int rcv_render_twostates(const rcv_scene *scene,
  * the shape of parameter param_ids[i]. Path replay: nothing is taped. The
  * volume integrators' adjoints (samples_per_thread 0) log density
  * scatter-adds in a buffer that the library allocates on first use per
- * (device, stream), about 3.3 GB, and keeps until the process ends; calls on
+ * (device, stream), about 3.2 GB, and keeps until the process ends; calls on
  * one stream share it in stream order. A captured call adds with atomics. */
 int rcv_render_backward(const rcv_scene *scene,
                         const rcv_integrator_desc *integrator, int32_t sensor,
@@ -355,7 +355,13 @@ int rcv_batch_create(rcv_batch **out);
 int rcv_batch_destroy(rcv_batch *batch);
 int rcv_batch_add_job(rcv_batch *batch, const rcv_batch_job *job, int32_t *out_job);
 /* Lays the jobs out in device memory; the scenes' parameter states must be
- * bound to param_ring[0] (OLD) and param_ring[1] (NEW) beforehand. */
+ * bound to param_ring[0] (OLD) and param_ring[1] (NEW) beforehand. A batch with
+ * jobs that optimise the density of a medium in a box, on a grid of up to
+ * 262144 voxels, logs their scatter-adds in a buffer of about 3.2 GB of its
+ * own, taken here and handed to the next batch when this one is destroyed
+ * (one is kept per device until the process ends; without memory for it the
+ * batch adds with atomics). A batch made before the last one is destroyed
+ * takes a second one. */
 int rcv_batch_commit(rcv_batch *batch, void *stream);
 /* Launch shape of the persistent kernels: threads per block (64..512, a
  * multiple of 64, and at most what the device's LDS per block holds at 160 B

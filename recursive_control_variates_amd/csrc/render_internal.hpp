@@ -56,10 +56,11 @@ constexpr int kWavesPerEu = INTEG == RCV_INTEGRATOR_VOLPATH ? 4 : 3;
 // spills) they run 12-14 % / 17-18 % faster over the optimisation (two
 // waves: no faster than three). That holds for the adjoint whose density
 // gradient goes through the scatter log; adjoints that add with device-scope
-// atomics (batched, static, grids past the log) are faster at four, whose
-// extra wave covers the atomics' waits (the 64-job batch: 348 ms per
-// iteration against 376 ms with its adjoint at three). The single-state
-// render stays at four.
+// atomics (static, in batches, of grids past the log) are faster at four,
+// whose extra wave covers the atomics' waits (64 volume jobs in a batch on
+// these kernels: 348 ms per iteration against 376 ms with the adjoint at
+// three). The single-state render stays at four. (All of the general kernels;
+// the one-box tracker's wave count is kBoxWaves.)
 template <int NS, int INTEG>
 constexpr int kWavesPerEuRender = INTEG == RCV_INTEGRATOR_VOLPATH && NS == 2 ? 3 : kWavesPerEu<INTEG>;
 constexpr int kWavesPerEuLoggedAdjoint = 3;
@@ -95,9 +96,13 @@ __host__ __device__ inline int sample_end(int c, int spp, int chunk_log2) {
 // launches (the adjoint; the renders, within kRenderMaxUnitsPerPixel). With
 // small units the lanes of a wavefront trace samples of the same few pixels,
 // whose paths start alike and share L1 lines of the grid, and the last units
-// of a launch are short. The 64^3 adjoint at the mid / final state of the
-// optimisation: 46.1 / 67.5 ms with 16-sample units, 39.7 / 51.4 with 8,
-// 37.0 / 47.8 with 4, 36.2 / 46.4 with 2.
+// of a launch are short. The general kernels' 64^3 adjoint at the mid / final
+// state of the optimisation: 46.1 / 67.5 ms with 16-sample units, 39.7 / 51.4
+// with 8, 37.0 / 47.8 with 4, 36.2 / 46.4 with 2. On the one-box tracker, units
+// of 16, 8, 4, 2 and 1: the 64^3 step (4 x 256^2, 32 samples) 16.3, 13.4, 12.2,
+// 11.4 and 11.1 ms; the 128^3 step with an albedo grid 7.7 ms from 2 on, 7.1
+// with 1; 64^3 with a supergrid and volpathsimple's adjoint 5.4 ms from 2 on,
+// 4.7 with 1.
 constexpr int kVolUnitSamples = 2;
 
 // Render, adjoint and forward mode of the one-box volume tracker.
@@ -106,8 +111,12 @@ constexpr int kBoxAdjoint = 1;
 constexpr int kBoxForward = 2;
 
 // Waves per SIMD of the one-box volume tracker (boxpath.hpp): four, up to 128
-// VGPRs. It is bound by instruction issue; three and five waves measured
-// within 3 % of four.
+// VGPRs, within which all variants but the two-state renders with an albedo
+// grid fit. It is bound by instruction issue: at three, four and five waves the
+// 64^3 step takes 11.3, 11.5 and 11.5 ms, the 128^3 render 3.76, 3.77 and 3.80.
+// The two-state render spills 44 bytes per lane at four with an albedo grid, 72
+// with a supergrid besides: the 128^3 step with an albedo grid 7.1 ms at three
+// (no spills), 7.7 at four, 8.6 at five.
 template <int NS, int MODE>
 constexpr int kBoxWaves = 4;
 
@@ -149,7 +158,8 @@ inline bool takes_simple_box(const Scene *s, const rcv_integrator_desc *d) {
 }
 
 // Waves per SIMD of volpathsimple's adjoint on the tracker: four, which its
-// LDS allows (64^3 step: 6.61 ms, with three 6.61 ms).
+// LDS allows (64^3 with a supergrid: the step 5.34 ms, at three 5.36, at five
+// 5.75). With an albedo grid it spills 48 to 80 bytes per lane at four.
 constexpr int kSimpleBoxWaves = 4;
 
 // Calls fn with the compile-time feature mask of a one-box scene.

@@ -18,8 +18,8 @@
 // 64^3 grid, 128^2, 16 samples, majorant supergrid: 3.45 ms against 6.1 ms of
 // the nested loops (both logged, and 0.5 ms of reduction); a 64^2 call of 4
 // samples on 32^3, which waits for its longest path, 1.06 against 1.12 ms.
-// Bound by instruction issue: a tracking step walks the supergrid's cells one
-// by one. With events run at half, one, two and three times as many waiting
+// Bound by instruction issue with 13 % of the lanes active: a tracking step
+// walks the supergrid's cells one by one. With events run at half, one, two and three times as many waiting
 // as tracking lanes the step takes 7.03, 6.64, 6.51 and 6.73 ms.
 #pragma once
 

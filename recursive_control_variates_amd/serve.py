@@ -76,7 +76,10 @@ def make_job(seed: int, kind: str, method: str = "cv_ps", device="cuda", spp_ref
 def footprint_estimate(meta) -> int:
     """Device bytes a job will hold: parameter ring x3 + Adam m, v + gradient
     (6 parameter-sized arrays) and 13 image-sized arrays (reference, H, F,
-    image, image gradient, 8 CV arrays), plus a fixed 1 MiB for the scene."""
+    image, image gradient, 8 CV arrays), plus a fixed 1 MiB for the scene.
+    Beside the jobs a batch with volume jobs holds a scatter log of 3.2 GB,
+    once per device whatever their number; leave room for it when choosing a
+    budget."""
     n_param = meta["grid"] ** 3 if meta["kind"] == "volume" else 64 * 64 * 3
     n_img = meta["side"] * meta["side"] * 3
     return 4 * (6 * n_param + 13 * n_img) + (1 << 20)
