@@ -17,8 +17,9 @@
  *     scratch (96 bytes per pixel of the largest sensor, for a small image of a
  *     medium in a box more, 6 MB at most; allocated at its first call, kept
  *     until the scene is destroyed; past 32 streams a new one waits for the
- *     device and takes over another's). Captured launches of a scene share one more: graphs that
- *     hold renders or adjoints of one scene must not run at the same time.
+ *     device and takes over another's). Captured launches of a
+ *     scene share one more: graphs that hold renders or adjoints of one scene
+ *     must not run at the same time, nor may two of them within a graph.
  *   - A CV state is not re-entrant: two rcv_cv_step calls on one state must be
  *     ordered on one stream.
  *   - Images are row-major (height, width, 3) float32. Textures are

@@ -62,6 +62,16 @@ inline bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
+// Within its life the calling thread's allocations and synchronisations do not
+// break off the captures under way (its own or, in global mode, any thread's).
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+  RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+};
+
 inline bool aligned16(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

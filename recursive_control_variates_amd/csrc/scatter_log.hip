@@ -312,6 +312,7 @@ __global__ void zero_ctl_kernel(unsigned *p) { p[threadIdx.x] = 0u; }
 constexpr int kCtlWords = 1 + kLogBins;
 
 int allocate(LogBuf &out) {
+  const RelaxedCapture relaxed;
   LogBuf nb;
   hipError_t e = hipMalloc(&nb.rec, size_t(kLogPool) * kLogChunk * sizeof(float4));
   if (e == hipSuccess) e = hipMalloc(&nb.ctl, kCtlWords * sizeof(unsigned));

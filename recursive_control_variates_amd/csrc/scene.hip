@@ -550,13 +550,10 @@ int Scene::upload(hipStream_t stream) {
 }
 
 int Scene::add_scratch(hipStream_t stream, bool captured) const {
-  // an allocation breaks off captures of its thread, unless it is told not to mind them
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  RCV_TRY_HIP(hipThreadExchangeStreamCaptureMode(&mode), "launch scratch: capture mode");
+  const RelaxedCapture relaxed;
   void *p = nullptr;
   const size_t sums = size_t(partial_cap) * sizeof(float);
   const hipError_t e = hipMalloc(&p, sums + 256);
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return hip_fail(e, "launch scratch: hipMalloc");
@@ -580,7 +577,10 @@ int Scene::scratch(hipStream_t stream, bool captured, LaunchScratch &out) const 
     }
   }
   if (!own && oldest && (!oldest->used || streams >= kMaxScratchStreams)) {
-    if (oldest->used) RCV_TRY_HIP(hipDeviceSynchronize(), "launch scratch: synchronize");
+    if (oldest->used) {
+      const RelaxedCapture relaxed;
+      RCV_TRY_HIP(hipDeviceSynchronize(), "launch scratch: synchronize");
+    }
     oldest->stream = stream;
     own = oldest;
   }

@@ -1,5 +1,7 @@
 """Calls on one scene from several streams, and captured calls replayed
 beside eager ones."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -7,6 +9,7 @@ import torch
 import recursive_control_variates_amd as rcv
 from conftest import announce
 from helpers import homogeneous_box_scene, volume_box_scene
+from recursive_control_variates_amd import _native as N
 
 pytestmark = pytest.mark.gpu
 
@@ -146,3 +149,27 @@ def test_captured_adjoint_after_an_eager_one(cuda, kind):
         torch.cuda.synchronize()
         _assert_close(name, out, want)
         _assert_close(name, beside, want_other)
+
+
+def test_first_call_on_a_stream_while_another_is_captured(cuda):
+    # its scratch and its scatter log are allocated then, which leaves the
+    # capture as it is
+    announce("first adjoint on a stream while another stream is being captured")
+    sc, p, key, gimg, _ = _scene()
+    integ = rcv.load_dict({"type": "prbvolpath", "max_depth": 8, "rr_depth": 4})
+    want = integ.adjoint(sc, p, gimg, 0, 500, SPP)[key]
+    got, d, index = torch.zeros_like(want), integ.desc(), N.i32_array([sc.params[key].index])
+    grads = (C.c_void_p * 1)(got.data_ptr())
+    x = torch.zeros(1000, device="cuda")
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        x.add_(1.0)
+        N.call("rcv_render_backward", sc.handle, C.byref(d), 0, C.c_uint32(500), SPP, C.c_void_p(gimg.data_ptr()), 1,
+               index, grads, C.c_void_p(other.cuda_stream))
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert float(x.min()) == float(x.max()) == 3.0
+    _assert_close("adjoint", got, want)
